@@ -302,6 +302,29 @@ W4A8_API int w4a8_moe_forward_noalloc(const void* x, int x_dtype, int64_t T, int
                                       int64_t num_global_experts, float* topk_weights,
                                       int32_t* topk_ids, void* out, void* stream);
 
+/* Activations of w4a8_moe_mxfp4_apply. */
+#define W4A8_ACT_SILU 0        /* silu(gate) * up, w13 rows [gate | up] */
+#define W4A8_ACT_SWIGLUOAI 1   /* gpt-oss swigluoai, w13 rows interleaved (gate, up, gate, ...) */
+
+/* A whole MoE layer on E2M1 (mxfp4) weights with fp16 scales per 32 weights, optional fp16
+ * per-expert biases w13_bias (E, 2*inter) and w2_bias (E, H) (NULL: none), and the gated
+ * activation between the GEMMs (alpha and limit are swigluoai's): align, act-quant, gemm1 +
+ * bias + activation, act-quant, gemm2 + bias, weighted reduce, each rounding point where the
+ * op-by-op composition has it (moe_experts.py:587-665, called by the mxfp4 hook
+ * moe_experts.py:1351-1450). H and inter are multiples of 32, at least 128; expert_map and
+ * num_global_experts as in w4a8_moe_apply. */
+W4A8_API size_t w4a8_moe_mxfp4_workspace_size(int64_t T, int64_t H, int64_t inter, int64_t E,
+                                              int64_t top_k);
+W4A8_API int w4a8_moe_mxfp4_apply(const void* x, int x_dtype, int64_t T, int64_t H, int64_t inter,
+                                  int64_t E, int64_t top_k, const int32_t* w13,
+                                  const void* w13_scales_f16, const void* w13_bias_f16,
+                                  const int32_t* w2, const void* w2_scales_f16,
+                                  const void* w2_bias_f16, int activation, float alpha,
+                                  float limit, const float* topk_weights,
+                                  const int32_t* topk_ids, const int32_t* expert_map,
+                                  int64_t num_global_experts, void* out, int out_dtype,
+                                  void* workspace, size_t workspace_bytes, void* stream);
+
 /* Optional per-stage timing of the whole-layer calls on the calling thread: when count >= 8,
  * the next w4a8_moe_apply / _fragments / w4a8_moe_forward calls record events[0] before the
  * first expert-path launch and events[i] after stage i (1 align, 2 act-quant x, 3 reserved

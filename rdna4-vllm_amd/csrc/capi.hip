@@ -561,6 +561,51 @@ int moe_apply_impl(const void* x, int x_dtype, int64_t T, int64_t H, int64_t int
 namespace w4a8 {
 namespace {
 
+// ---- mxfp4 layer (w4a8_moe_mxfp4_apply) ----
+struct MxPlan {
+    int64_t block_m, P, nblk;
+};
+// 16-row tiles while an expert has fewer than 8 slots on average, so few of them pass 16;
+// past that more and more experts fill several 16-row blocks, each streaming the expert's
+// weights (gemm1 at 2880 x 5760, 32 experts, top-4, 16- against 64-row tiles: T = 8 45 / 50 us,
+// T = 64 82 / 83, T = 100 94 / 88, T = 256 160 / 98)
+MxPlan plan_mxfp4(int64_t T, int64_t E, int64_t top_k) {
+    MxPlan pl;
+    pl.block_m = T * top_k < 8 * E ? 16 : 64;
+    pl.P = w4a8_moe_align_sorted_len(T * top_k, E, pl.block_m);
+    pl.nblk = pl.P / pl.block_m;
+    return pl;
+}
+struct MxScratch {
+    int32_t *sti, *eid, *ntp, *s2r;
+    void* align_ws;
+    size_t align_bytes;
+    uint8_t *xq, *hq;
+    float *s1, *s2;
+    __half *h, *y;
+};
+template <typename WS>
+void carve_mxfp4(WS& w, const MxPlan& pl, int64_t T, int64_t H, int64_t inter, int64_t E,
+                 int64_t top_k, MxScratch& m) {
+    m.sti = w.template take<int32_t>((size_t)pl.P);
+    m.eid = w.template take<int32_t>((size_t)pl.nblk);
+    m.ntp = w.template take<int32_t>(1);
+    m.s2r = w.template take<int32_t>((size_t)(T * top_k));
+    m.align_bytes = align_workspace_bytes(T * top_k, E);
+    m.align_ws = w.template take<uint8_t>(m.align_bytes);
+    m.xq = w.template take<uint8_t>((size_t)(T * H));
+    m.s1 = w.template take<float>((size_t)T);
+    m.h = w.template take<__half>((size_t)(pl.P * inter));
+    m.hq = w.template take<uint8_t>((size_t)(pl.P * inter));
+    m.s2 = w.template take<float>((size_t)pl.P);
+    m.y = w.template take<__half>((size_t)(pl.P * H));
+}
+struct MxSizeProbe {
+    WorkspaceSize s;
+    template <typename T>
+    T* take(size_t n) { s.take<T>(n); return nullptr; }
+};
+
 // Scratch of w4a8_moe_forward_noalloc: device data of the code object, one copy per GPU,
 // allocated when the library's code is loaded onto that GPU and held until the process
 // ends. In host code the array's name is only a stand-in for the symbol; the device address
@@ -925,6 +970,73 @@ int w4a8_moe_forward_noalloc(const void* x, int x_dtype, int64_t T, int64_t H, i
                             renormalize, w13, w13_scales_f16, w13_zeros, w2, w2_scales_f16,
                             w2_zeros, weights_layout, expert_map, num_global_experts,
                             topk_weights, topk_ids, out, ws, w4a8::kNoAllocScratchBytes, stream);
+}
+
+size_t w4a8_moe_mxfp4_workspace_size(int64_t T, int64_t H, int64_t inter, int64_t E,
+                                     int64_t top_k) {
+    MxSizeProbe sp;
+    MxScratch m;
+    carve_mxfp4(sp, plan_mxfp4(T, E, top_k), T, H, inter, E, top_k, m);
+    return sp.s.used;
+}
+
+int w4a8_moe_mxfp4_apply(const void* x, int x_dtype, int64_t T, int64_t H, int64_t inter,
+                         int64_t E, int64_t top_k, const int32_t* w13, const void* w13_scales_f16,
+                         const void* w13_bias_f16, const int32_t* w2, const void* w2_scales_f16,
+                         const void* w2_bias_f16, int activation, float alpha, float limit,
+                         const float* topk_weights, const int32_t* topk_ids,
+                         const int32_t* expert_map, int64_t num_global_experts, void* out,
+                         int out_dtype, void* workspace, size_t workspace_bytes, void* stream) {
+    clear_error();
+    W4A8_REQUIRE(x_dtype == W4A8_DTYPE_F16 || x_dtype == W4A8_DTYPE_BF16, "x dtype must be fp16 or bf16");
+    W4A8_REQUIRE(out_dtype == W4A8_DTYPE_F16 || out_dtype == W4A8_DTYPE_BF16, "out dtype must be fp16 or bf16");
+    W4A8_REQUIRE(activation == W4A8_ACT_SILU || activation == W4A8_ACT_SWIGLUOAI,
+                 "moe_mxfp4_apply: activation must be W4A8_ACT_SILU or W4A8_ACT_SWIGLUOAI");
+    W4A8_REQUIRE(T >= 0 && H > 0 && inter > 0 && E > 0 && top_k > 0, "moe_mxfp4_apply: invalid sizes");
+    const MxPlan pl = plan_mxfp4(T, E, top_k);
+    W4A8_REQUIRE(fp4_tiles_supported(T, H, 2 * inter, 32, true) &&
+                 fp4_tiles_supported(pl.P, inter, H, 32, true),
+                 "moe_mxfp4_apply: hidden and intermediate sizes must be multiples of 32, at least 128, "
+                 "expert slices and rows below 2 GiB");
+    if (num_global_experts <= 0) num_global_experts = E;
+    W4A8_REQUIRE(expert_map != nullptr || num_global_experts == E,
+                 "moe_mxfp4_apply: global expert count differs from the local one; pass expert_map");
+    W4A8_REQUIRE(num_global_experts <= (int64_t)1 << 20, "moe_mxfp4_apply: too many global experts");
+    if (T == 0) return W4A8_OK;
+    W4A8_REQUIRE(x && w13 && w13_scales_f16 && w2 && w2_scales_f16 && topk_weights && topk_ids && out,
+                 "moe_mxfp4_apply: null pointer");
+    Workspace w(workspace, workspace_bytes);
+    MxScratch m;
+    carve_mxfp4(w, pl, T, H, inter, E, top_k, m);
+    if (workspace == nullptr || !w.ok()) {
+        set_error("moe_mxfp4_apply: workspace smaller than w4a8_moe_mxfp4_workspace_size()");
+        return W4A8_ERR_WORKSPACE;
+    }
+    hipStream_t s = as_stream(stream);
+    const int64_t numel = T * top_k;
+    if (int rc = launch_align(topk_ids, numel, E, pl.block_m, expert_map, num_global_experts, m.sti,
+                              pl.P, m.eid, m.ntp, m.align_ws, m.align_bytes, s, m.s2r))
+        return rc;
+    if (int rc = launch_act_quant(x, x_dtype == W4A8_DTYPE_BF16, T, H, m.xq, m.s1, false, s))
+        return rc;
+    GroupedArgs g1{};
+    g1.x_rows = T; g1.K = H; g1.w = w13; g1.scales = static_cast<const uint16_t*>(w13_scales_f16);
+    g1.E = E; g1.N = 2 * inter; g1.group_size = 32; g1.sorted_ids = m.sti; g1.P = pl.P;
+    g1.expert_ids = m.eid; g1.ntp = m.ntp; g1.top_k = top_k; g1.num_valid = numel;
+    g1.block_m = pl.block_m; g1.e2m1 = true; g1.out_top_k = top_k; g1.out = m.h;
+    g1.epi = activation == W4A8_ACT_SILU ? Epi::kSiluHalf : Epi::kSwigluHalf;
+    g1.x_fp8 = m.xq; g1.act_scales = m.s1; g1.bias = w13_bias_f16; g1.alpha = alpha; g1.limit = limit;
+    if (int rc = launch_grouped_fp4(g1, s)) return rc;
+    // real rows of h only
+    if (int rc = launch_act_quant(m.h, false, pl.P, inter, m.hq, m.s2, false, s, m.sti, m.ntp, numel))
+        return rc;
+    GroupedArgs g2 = g1;
+    g2.x_rows = pl.P; g2.K = inter; g2.w = w2; g2.scales = static_cast<const uint16_t*>(w2_scales_f16);
+    g2.N = H; g2.identity_gather = true; g2.out = m.y; g2.epi = Epi::kHalf; g2.x_fp8 = m.hq;
+    g2.act_scales = m.s2; g2.bias = w2_bias_f16;
+    if (int rc = launch_grouped_fp4(g2, s)) return rc;
+    return launch_row_reduce(m.y, m.s2r, topk_weights, T, H, top_k, out,
+                             out_dtype == W4A8_DTYPE_BF16, s);
 }
 
 int w4a8_set_decode_fused(int on) {

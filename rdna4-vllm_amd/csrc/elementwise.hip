@@ -67,12 +67,7 @@ __global__ void swigluoai_and_mul_kernel(const __half* __restrict__ in, int64_t 
     const int64_t r = i / inter;
     const int c = (int)(i % inter);
     const __half2 gu = *reinterpret_cast<const __half2*>(in + r * 2 * inter + 2 * c);
-    const float gate = __low2float(gu), up = __high2float(gu);
-    const float g = gate > limit ? limit : gate;
-    const float u = up > limit ? limit : (up < -limit ? -limit : up);
-    const float sig = 1.0f / (1.0f + expf(as_f32(-g * alpha)));
-    const float glu = as_f32(g * sig);
-    out[i] = __float2half(as_f32((u + 1.0f) * glu));
+    out[i] = swigluoai_h(__low2half(gu), __high2half(gu), alpha, limit);
 }
 
 __global__ void inverse_map_kernel(const int32_t* __restrict__ sorted_ids,

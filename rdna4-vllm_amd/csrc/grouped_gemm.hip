@@ -13,7 +13,8 @@
 //                            straight from HBM into MFMA B fragments (no LDS, no barriers)
 //                            with several groups of loads in flight (replaces
 //                            moe_kernel.hip:884-1062).
-// All read prequantised activations: x_fp8 rows in k8-interleaved order + act_scales.
+// All read prequantised activations: x_fp8 rows in k8-interleaved order + act_scales (E2M1 on
+// the matrix cores: natural order; with groups of 32 they run fp4_tiles.hip).
 #include <algorithm>
 #include <type_traits>
 
@@ -1008,6 +1009,7 @@ int launch_grouped_scalar(const GroupedArgs& a, hipStream_t s) {
         case Epi::kSiluHalf: return launch_scalar_t<Epi::kSiluHalf>(p, s);
         case Epi::kScatter: return launch_scalar_t<Epi::kScatter>(p, s);
         case Epi::kSlotF32: return launch_scalar_t<Epi::kSlotF32>(p, s);
+        case Epi::kSwigluHalf: break;   // E2M1 tiles only
     }
     return W4A8_ERR_INVALID;
 }
@@ -1019,12 +1021,16 @@ int launch_grouped_mfma(const GroupedArgs& a, hipStream_t s) {
         set_error("mfma grouped GEMM reads op-layout weights only");
         return W4A8_ERR_INVALID;
     }
+    // mxfp4's own group size: fp4 operands with block scales
+    if (fp4_tiles_supported(a.x_rows, a.K, a.N, a.group_size, a.e2m1)) return launch_grouped_fp4(a, s);
     switch (a.epi) {
+        case Epi::kSwigluHalf: break;   // E2M1 groups of 32 only
         case Epi::kHalf: return launch_mfma_e<Epi::kHalf>(p, s);
         case Epi::kSiluHalf: return launch_mfma_e<Epi::kSiluHalf>(p, s);
         case Epi::kScatter: return launch_mfma_e<Epi::kScatter>(p, s);
         case Epi::kSlotF32: return launch_mfma_e<Epi::kSlotF32>(p, s);
     }
+    set_error("mfma grouped GEMM: the swigluoai epilogue needs E2M1 weights with groups of 32");
     return W4A8_ERR_INVALID;
 }
 
@@ -1052,6 +1058,7 @@ int launch_grouped_gemv_tpt(const GroupedArgs& a, int tpt, hipStream_t s) {
         case Epi::kSiluHalf: return launch_gemv_e<Epi::kSiluHalf>(p, tpt, s);
         case Epi::kScatter: return launch_gemv_e<Epi::kScatter>(p, tpt, s);
         case Epi::kSlotF32: return launch_gemv_e<Epi::kSlotF32>(p, tpt, s);
+        case Epi::kSwigluHalf: break;   // E2M1 tiles only
     }
     return W4A8_ERR_INVALID;
 }

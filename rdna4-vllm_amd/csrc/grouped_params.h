@@ -37,6 +37,8 @@ struct Params {
     int xbf16;                  // xh holds bf16 (else fp16)
     int w_frag;                 // w in fragment layout (16-row tile, group, lane)
     const float* asum;          // (x_rows, K/128) sums of the e4m3 values per group, or null
+    const __half* bias;         // (E, N) or null (E2M1 tiles)
+    float alpha, limit;         // swigluoai (E2M1 tiles)
     int xcd_slots;              // activation-resident tiles: work-groups one XCD runs at once
 };
 
@@ -77,6 +79,9 @@ inline Params make_params(const GroupedArgs& a) {
     p.xbf16 = a.x_bf16 ? 1 : 0;
     p.asum = a.act_group_sums;
     p.w_frag = a.w_frag ? 1 : 0;
+    p.bias = static_cast<const __half*>(a.bias);
+    p.alpha = a.alpha;
+    p.limit = a.limit;
     p.xcd_slots = 0;
     return p;
 }

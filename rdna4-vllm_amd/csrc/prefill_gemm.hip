@@ -443,6 +443,7 @@ int launch_grouped_prefill(const GroupedArgs& a, hipStream_t s) {
         case Epi::kSiluHalf: return launch_prefill_e<Epi::kSiluHalf>(p, s);
         case Epi::kScatter: return launch_prefill_e<Epi::kScatter>(p, s);
         case Epi::kSlotF32: return launch_prefill_e<Epi::kSlotF32>(p, s);
+        case Epi::kSwigluHalf: break;   // E2M1 tiles only
     }
     return W4A8_ERR_INVALID;
 }

@@ -273,6 +273,17 @@ __device__ __forceinline__ __half silu_mul_h(__half gate_h, __half up_h) {
     return __hmul(silu_h(gate_h), up_h);
 }
 
+// gpt-oss gated activation of one fp16 (gate, up) pair: in fp32, g = min(gate, limit),
+// u = clamp(up, -limit, limit), fp16((u + 1) * (g * (1 / (1 + exp(-g * alpha))))).
+__device__ __forceinline__ __half swigluoai_h(__half gate_h, __half up_h, float alpha, float limit) {
+    const float gate = __half2float(gate_h), up = __half2float(up_h);
+    const float g = gate > limit ? limit : gate;
+    const float u = up > limit ? limit : (up < -limit ? -limit : up);
+    const float sig = 1.0f / (1.0f + expf(as_f32(-g * alpha)));
+    const float glu = as_f32(g * sig);
+    return __float2half(as_f32((u + 1.0f) * glu));
+}
+
 // silu_mul_h of four (gate, up) pairs given as fp32 values (each rounded to fp16 first): the
 // fast form of all four first, so that their chains interleave, then the exact form of those
 // it does not cover (each a branch that the wave skips unless one of its lanes needs it).

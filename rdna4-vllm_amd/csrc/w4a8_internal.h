@@ -141,6 +141,7 @@ enum class Epi : int {
     kSiluHalf = 1,  // out[row_pad, n] = silu_mul(gate, up)          (P, N/2)
     kScatter = 2,   // atomicAdd(out[slot / top_k, n], w[slot] * run * asc)
     kSlotF32 = 3,   // out[slot, n] = run * asc (fp32, rows = M*top_k)
+    kSwigluHalf = 4,  // out[row_pad, n] = swigluoai(row 2n, row 2n + 1)  (P, N/2); E2M1 tiles
 };
 
 struct GroupedArgs {
@@ -170,6 +171,10 @@ struct GroupedArgs {
     uint8_t* x_fp8;         // (x_rows, K) k8-interleaved, or null
     float* act_scales;      // (x_rows,)
     float* act_group_sums;  // (x_rows, K/128) per-group sums of the e4m3 values, or null
+    // E2M1 tiles (launch_grouped_fp4): fp16 bias (E, N) added to the fp16 result of the GEMM,
+    // before the activation, or null; swigluoai parameters (kSwigluHalf)
+    const void* bias;
+    float alpha, limit;
 };
 
 // Dense GEMV for 1 <= M <= 16 rows of fp16 x on op-layout weights (dense_gemv.hip): group
@@ -179,6 +184,10 @@ int launch_dense_gemv(const void* x_f16, int64_t M, int64_t K, const int32_t* w,
                       const int32_t* zeros, int64_t N, void* out_f16, hipStream_t s);
 int launch_grouped_scalar(const GroupedArgs& a, hipStream_t stream);
 int launch_grouped_mfma(const GroupedArgs& a, hipStream_t stream);   // prefill tiles
+// E2M1 weights with groups of 32 on fp4 MFMA operands with block scales (fp4_tiles.hip); rows
+// quantised in natural k order.
+bool fp4_tiles_supported(int64_t x_rows, int64_t K, int64_t N, int64_t group_size, bool e2m1);
+int launch_grouped_fp4(const GroupedArgs& a, hipStream_t stream);
 int launch_grouped_gemv(const GroupedArgs& a, hipStream_t stream);   // decode GEMV
 // Prefill, activation-resident schedule (prefill_ares.hip): 64-row tiles, all N per tile.
 bool prefill_ares_supported(int64_t K, int64_t N, int64_t group_size, bool e2m1, int64_t block_m,

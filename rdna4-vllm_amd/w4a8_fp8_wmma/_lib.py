@@ -73,6 +73,12 @@ SIGNATURES = {
                                         _c_void_p, _int, _c_void_p, _c_void_p, _c_void_p,
                                         _c_void_p, _c_void_p, _c_void_p, _int, _c_void_p, _i64,
                                         _c_void_p, _c_void_p, _c_void_p, _c_void_p]),
+    "w4a8_moe_mxfp4_workspace_size": (_size, [_i64, _i64, _i64, _i64, _i64]),
+    "w4a8_moe_mxfp4_apply": (_int, [_c_void_p, _int, _i64, _i64, _i64, _i64, _i64, _c_void_p,
+                                    _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _int,
+                                    ctypes.c_float, ctypes.c_float, _c_void_p, _c_void_p,
+                                    _c_void_p, _i64, _c_void_p, _int, _c_void_p, _size,
+                                    _c_void_p]),
     "w4a8_set_decode_fused": (_int, [_int]),
     "w4a8_set_prefill_pair": (_int, [_int]),
     "w4a8_decode_fused_test_fault": (_int, [_int]),

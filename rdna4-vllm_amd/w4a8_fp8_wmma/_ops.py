@@ -539,6 +539,58 @@ def moe_forward(x, router_logits, top_k: int, w13, w2, w13_s, w2_s, w13_z, w2_z,
     return out, tw, ids
 
 
+def mxfp4_layer_supported(slots, w13, w2, w13_s, w2_s, w13_b, w2_b, n_global, expert_map) -> bool:
+    """Whether moe_apply_mxfp4 takes these op-layout E2M1 tensors: groups of 32, hidden and
+    intermediate sizes of at least 128, whole (E, N) biases, contiguous weights and scales, an
+    expert count that the map (or, without one, the weights) agrees with, and sizes that 32-bit
+    offsets reach (slots: tokens times top_k)."""
+    if w13.dim() != 3 or w2.dim() != 3 or w13_s.dim() != 3 or w2_s.dim() != 3:
+        return False
+    E, N, kw = w13.shape
+    H, inter = kw * 8, N // 2
+    return (N % 2 == 0 and H >= 128 and inter >= 128 and H % 32 == 0 and inter % 32 == 0
+            and w13.dtype == torch.int32 and w2.dtype == torch.int32
+            and w13_s.dtype == torch.float16 and w2_s.dtype == torch.float16
+            and tuple(w2.shape) == (E, H, inter // 8)
+            and tuple(w13_s.shape) == (E, N, H // 32) and tuple(w2_s.shape) == (E, H, inter // 32)
+            and (w13_b is None or tuple(w13_b.shape) == (E, N))
+            and (w2_b is None or tuple(w2_b.shape) == (E, H))
+            and all(t.is_contiguous() for t in (w13, w2, w13_s, w2_s))
+            and (slots + 64 * E) * max(H, inter) < 1 << 31 and inter * H < 1 << 31
+            and n_global == (E if expert_map is None else expert_map.numel()))
+
+
+def moe_apply_mxfp4(x, w13, w2, w13_s, w2_s, w13_b, w2_b, topk_weights, topk_ids, activation,
+                    expert_map, n_global, out_dtype) -> torch.Tensor:
+    """Whole mxfp4 MoE layer in one C-ABI call, for tensors that mxfp4_layer_supported takes:
+    the bits of the op-by-op composition. x (T, H) fp16 / bf16 -> (T, H) in out_dtype."""
+    T, H = x.shape
+    E, N = w13.shape[:2]
+    top_k = topk_ids.shape[1]
+    if H != w13.shape[2] * 8:
+        _fail(f"x must be (T, {w13.shape[2] * 8})")
+    if topk_ids.shape[0] != T or topk_weights.numel() != T * top_k:
+        _fail(f"topk_weights and topk_ids must be (T, top_k) with T={T}")
+    x = x.contiguous()
+    tw = topk_weights.to(torch.float32).contiguous()
+    ids = topk_ids.to(torch.int32).contiguous()
+    b13 = None if w13_b is None else w13_b.to(torch.float16).contiguous()
+    b2 = None if w2_b is None else w2_b.to(torch.float16).contiguous()
+    emap = None if expert_map is None else expert_map.to(device=x.device, dtype=torch.int32).contiguous()
+    for t in (x, w13, w2, w13_s, w2_s, tw, ids, b13, b2):
+        if t is not None and (not t.is_cuda or t.device != x.device):
+            _fail("all tensors must be CUDA tensors on x's device")
+    ws = _workspace(lib.w4a8_moe_mxfp4_workspace_size(T, H, N // 2, E, top_k), x.device)
+    out = torch.empty((T, H), dtype=out_dtype, device=x.device)
+    check(lib.w4a8_moe_mxfp4_apply(
+        _ptr(x), 1 if x.dtype == torch.bfloat16 else 0, T, H, N // 2, E, top_k, _ptr(w13),
+        _ptr(w13_s), _ptr(b13), _ptr(w2), _ptr(w2_s), _ptr(b2),
+        0 if activation == "silu" else 1, SWIGLUOAI_ALPHA, SWIGLUOAI_LIMIT, _ptr(tw), _ptr(ids),
+        _ptr(emap), n_global, _ptr(out), 1 if out_dtype == torch.bfloat16 else 0, ws.data_ptr(),
+        ws.numel(), _stream(x)), "moe_apply_mxfp4")
+    return out
+
+
 def fragments_supported(hidden: int, inter: int, group_size: int) -> bool:
     """Whether moe_apply takes fragment-layout weights of this shape for every batch size
     (what a load hook checks before it repacks)."""

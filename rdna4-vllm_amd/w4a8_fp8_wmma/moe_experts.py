@@ -301,6 +301,19 @@ def _run_grouped_moe(x, w1, w2, w1_s, w2_s, w1_zp, w2_zp,
         tw = topk_weights.to(torch.float32)
     ids = topk_ids.to(torch.int32)
 
+    # mxfp4 layers in one native call (the same bits as the composition below; a block_m set in
+    # the environment asks for the composition)
+    if (weight_is_e2m1 and kernel != "scalar" and env.block_m is None
+            and (w1_bias is not None or w2_bias is not None or act != "silu")
+            and w1_zp is None and w2_zp is None
+            and out_dtype in (torch.float16, torch.bfloat16)
+            and _ops.mxfp4_layer_supported(M * top_k, w1, w2, w1_s, w2_s, w1_bias, w2_bias,
+                                           global_num_experts, expert_map)):
+        if x.dtype not in (torch.float16, torch.bfloat16):
+            x = x.to(torch.float16)
+        return _ops.moe_apply_mxfp4(x, w1, w2, w1_s, w2_s, w1_bias, w2_bias, tw, ids, act,
+                                    expert_map, global_num_experts, out_dtype)
+
     if kernel == "scalar" or w1_bias is not None or w2_bias is not None or act != "silu":
         if w1.dim() == 4:   # the op-by-op kernels read the op layout
             w1, w2 = _fragments_to_op_layout(w1), _fragments_to_op_layout(w2)
