@@ -51,6 +51,14 @@ __device__ __forceinline__ void quantize_row_regs(const RowRegs& rr, int64_t row
                                                   float* __restrict__ scales, bool k8,
                                                   float* __restrict__ gsum, int lane);
 
+// A row of up to kBlockRowMaxK values by a work-group of four waves (row start 16-byte aligned):
+// wave w holds the 512-wide passes w, w + 4, ... in registers, the absmaxes meet in LDS.
+constexpr int kBlockRowMaxK = 16384;
+template <bool BF16>
+__device__ __forceinline__ void quantize_row_block(const void* __restrict__ x, int64_t row, int K,
+                                                   uint8_t* __restrict__ q, float* __restrict__ scales,
+                                                   bool k8, float* __restrict__ gsum, float* s_amax);
+
 // Group sum of one 512-wide pass (lanes 16j..16j+15 hold group k/128): fixed-order tree.
 __device__ __forceinline__ void row_group_sum(uint32_t lo, uint32_t hi, int64_t row, int K, int k,
                                               float* __restrict__ gsum, int lane) {
@@ -154,6 +162,71 @@ __device__ __forceinline__ void quantize_row_regs(const RowRegs& rr, int64_t row
                 hi = pack4_e4m3(f[4], f[5], f[6], f[7]);
             }
             *reinterpret_cast<uint2*>(q + base + k) = make_uint2(lo, hi);
+        }
+        if (gsum != nullptr) row_group_sum(lo, hi, row, K, k, gsum, lane);
+    }
+}
+
+// absmax of 8 values as the fp16-rounded fp32 value, NaNs not counted
+template <bool BF16>
+__device__ __forceinline__ float absmax_u4(const uint4& v) {
+    constexpr uint32_t nan_above = BF16 ? 0x7F80u : 0x7C00u;
+    using u16x2 = unsigned short __attribute__((ext_vector_type(2)));
+    const uint32_t wd[4] = {v.x, v.y, v.z, v.w};
+    u16x2 m2 = {0, 0};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2, wd[j] & 0x7FFF7FFFu));
+    const uint32_t mbits = max((uint32_t)m2.x, (uint32_t)m2.y);
+    if (__builtin_expect(mbits <= nan_above, 1)) return act_from_u4<BF16>(make_uint4(mbits, 0u, 0u, 0u), 0);
+    float amax = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(act_from_u4<BF16>(v, j)));
+    return amax;
+}
+
+template <bool BF16>
+__device__ __forceinline__ void quantize_row_block(const void* __restrict__ x, int64_t row, int K,
+                                                   uint8_t* __restrict__ q, float* __restrict__ scales,
+                                                   bool k8, float* __restrict__ gsum, float* s_amax) {
+    constexpr int kMaxPass = kBlockRowMaxK / 2048;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int npass = (K + 511) / 512;
+    const char* rowp = reinterpret_cast<const char*>(x) + row * K * 2;
+    uint4 v[kMaxPass];
+#pragma unroll
+    for (int u = 0; u < kMaxPass; ++u) {
+        const int k = (4 * u + wave) * 512 + lane * 8;
+        v[u] = make_uint4(0, 0, 0, 0);
+        if (4 * u + wave < npass && k < K) v[u] = *reinterpret_cast<const uint4*>(rowp + k * 2);
+    }
+    float amax = 0.0f;
+#pragma unroll
+    for (int u = 0; u < kMaxPass; ++u)
+        if (4 * u + wave < npass) amax = fmaxf(amax, absmax_u4<BF16>(v[u]));
+    amax = wave_max(amax);
+    if (lane == 0) s_amax[wave] = amax;
+    __syncthreads();
+    amax = fmaxf(fmaxf(s_amax[0], s_amax[1]), fmaxf(s_amax[2], s_amax[3]));
+    const float s = act_scale_from_absmax(amax);
+    if (threadIdx.x == 0) scales[row] = s;
+    const float inv = 1.0f / s;
+#pragma unroll
+    for (int u = 0; u < kMaxPass; ++u) {
+        if (4 * u + wave >= npass) break;                  // uniform over the wave
+        const int k = (4 * u + wave) * 512 + lane * 8;
+        uint32_t lo = 0, hi = 0;
+        if (k < K) {
+            float f[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) f[j] = act_from_u4<BF16>(v[u], j) * inv;
+            if (k8) {
+                lo = pack4_e4m3(f[0], f[2], f[4], f[6]);
+                hi = pack4_e4m3(f[1], f[3], f[5], f[7]);
+            } else {
+                lo = pack4_e4m3(f[0], f[1], f[2], f[3]);
+                hi = pack4_e4m3(f[4], f[5], f[6], f[7]);
+            }
+            *reinterpret_cast<uint2*>(q + row * K + k) = make_uint2(lo, hi);
         }
         if (gsum != nullptr) row_group_sum(lo, hi, row, K, k, gsum, lane);
     }
