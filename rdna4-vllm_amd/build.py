@@ -44,6 +44,7 @@ def hipcc() -> str:
 EXTRA_FLAGS = {
     "prefill_gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "prefill_ares.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "wide_tiles.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }
 
 

@@ -58,12 +58,19 @@ int check_grouped(int64_t rows, int64_t K, int64_t E, int64_t N, int64_t gs, int
 int run_grouped(GroupedArgs& a, int64_t kernel, void* ws, size_t ws_bytes, hipStream_t s) {
     const bool mfma = mfma_supported(a.K, a.group_size, a.e2m1);
     // E2M1 codebook weights take the matrix-core tiles (the GEMV feeds raw nibbles)
-    const bool gemv = gemv_supported(a.K, a.group_size) && !a.e2m1;
+    bool gemv = gemv_supported(a.K, a.group_size) && !a.e2m1;
+    // One expert on identity rows (the dense op) with fp16 out: the GEMV streams the weights once
+    // per 16 rows; past 16 row blocks of 1024 columns (or their product) the wide tiles lead (us,
+    // GEMV / 32 x 128 tiles: (N, K) = (4096, 4096) M = 64 19 / 23, M = 96 27 / 23; (8192, 4096)
+    // M = 32 20 / 23, M = 64 25 / 23; (12288, 4096) M = 17 28 / 22; (1024, 4096) M = 256 20 / 24)
+    const bool dense = a.E == 1 && a.expert_ids == nullptr && a.epi == Epi::kHalf && !a.w_frag &&
+                       wide_tiles_supported(a.x_rows, a.K, a.N, a.group_size, a.e2m1);
     Workspace w(ws, ws_bytes);
     a.x_fp8 = w.take<uint8_t>((size_t)(a.x_rows * a.K));
     a.act_scales = w.take<float>((size_t)a.x_rows);
     float* gsum = w.take<float>((size_t)(a.x_rows * ((a.K + 127) / 128)));
     const bool have_ws = !(a.x_rows > 0 && ws == nullptr) && w.ok();
+    if (dense && have_ws && (a.P + 15) / 16 * a.N > 16 * 1024) gemv = false;
     // identity-gathered inputs (gemm2 / scatter) have one row per padded row: skip padding.
     const bool filter = a.identity_gather && a.sorted_ids != nullptr;
     if (kernel == W4A8_MOE_KERNEL_GEMV && gemv) {
@@ -84,17 +91,21 @@ int run_grouped(GroupedArgs& a, int64_t kernel, void* ws, size_t ws_bytes, hipSt
         set_error("workspace smaller than w4a8_moe_gemm_workspace_size()");
         return W4A8_ERR_WORKSPACE;
     }
-    // gemv for K-group counts outside its split-K table runs the matrix-core tiles
+    // gemv for K-group counts outside its split-K table (or, dense, past its rows) runs the
+    // matrix-core tiles
     const bool tiles = (kernel == W4A8_MOE_KERNEL_WMMA || kernel == W4A8_MOE_KERNEL_GEMV) && mfma;
     // E2M1 tiles take fp4 operands against activations in natural k order; every other
     // kernel (the scalar one included) takes k8-interleaved activations
     const bool k8 = !(a.e2m1 && tiles);
     const bool prefill = tiles && prefill_supported(a.K, a.group_size, a.e2m1);
-    a.act_group_sums = prefill ? gsum : nullptr;
+    const bool wide = tiles && dense;
+    const bool split = wide && dense_split_leads(a.P, a.N, a.K);
+    a.act_group_sums = (prefill || wide) && !split ? gsum : nullptr;
     if (int rc = launch_act_quant(a.x, a.x_bf16, a.x_rows, a.K, a.x_fp8, a.act_scales, k8, s,
                                   filter ? a.sorted_ids : nullptr, filter ? a.ntp : nullptr,
                                   a.num_valid, a.act_group_sums))
         return rc;
+    if (wide) return split ? launch_dense_split(a, s) : launch_wide_tiles(a, s);
     // activation-resident tiles where the shape allows (the whole-layer prefill kernel, so
     // the op API and moe_apply share it), the streamed-K tiles otherwise. An ares work-group
     // owns all N columns of its rows, so one expert (the dense GEMM) fills the chip only with

@@ -182,6 +182,14 @@ struct GroupedArgs {
 bool dense_gemv_supported(int64_t M, int64_t N, int64_t K, int64_t group_size, bool e2m1);
 int launch_dense_gemv(const void* x_f16, int64_t M, int64_t K, const int32_t* w, const void* scales_f16,
                       const int32_t* zeros, int64_t N, void* out_f16, hipStream_t s);
+// Wide streamed-K tiles (wide_tiles.hip): op-layout int4 weights of group 128, any K, rows
+// prequantised with group sums, fp16 out.
+bool wide_tiles_supported(int64_t x_rows, int64_t K, int64_t N, int64_t group_size, bool e2m1);
+int launch_wide_tiles(const GroupedArgs& a, hipStream_t s);
+// The same shapes with K split over a work-group's waves (dense_split.hip): one expert, identity
+// rows; for some tens of rows.
+bool dense_split_leads(int64_t M, int64_t N, int64_t K);
+int launch_dense_split(const GroupedArgs& a, hipStream_t s);
 int launch_grouped_scalar(const GroupedArgs& a, hipStream_t stream);
 int launch_grouped_mfma(const GroupedArgs& a, hipStream_t stream);   // prefill tiles
 // E2M1 weights with groups of 32 on fp4 MFMA operands with block scales (fp4_tiles.hip); rows

@@ -1,0 +1,67 @@
+"""The dense op's wide tiles and its split-K kernel at the edges of their tiles and of their
+dispatch, against the float64 product of the same quantised operands.
+
+Products are exact and summed in fp32, then one rounding to fp16: half an fp16 ulp of the value
+(2^-11) plus the fp32 sums' rounding, which stays below 2^-11 of the largest output at these
+sizes: 2^-10 of the largest in all."""
+import pytest
+import torch
+
+import w4a8_fp8_wmma as W
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _case(M, N, K, asym, seed, dtype=torch.float16):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    w = torch.randint(-2**31, 2**31 - 1, (N, K // 8), generator=g, device=DEV, dtype=torch.int64).to(torch.int32)
+    s = (torch.rand((N, K // 128), generator=g, device=DEV) * 0.015 + 0.005).to(torch.float16)
+    z = (torch.randint(-2**31, 2**31 - 1, (N // 8, K // 128), generator=g, device=DEV,
+                       dtype=torch.int64).to(torch.int32) if asym else None)
+    x = torch.randn((M, K), generator=g, device=DEV).to(dtype)
+    return x, w, s, z
+
+
+def _e4m3(b):
+    return b.view(torch.float8_e4m3fn).to(torch.float32).double()
+
+
+def _ref(x, w, s, z):
+    q, sc = W.act_quant_fp8(x.to(torch.float16))
+    wd = _e4m3(W.dequant_fp8(w, 128, z)) * s.double().repeat_interleave(128, dim=1)
+    return (_e4m3(q) @ wd.t()) * sc.double()[:, None]
+
+
+def _check(x, w, s, z, kernel):
+    got = W.mmq_fp8_gemm(x, w, s, kernel=kernel, w_zeros=z).double()
+    ref = _ref(x, w, s, z)
+    assert float((got - ref).abs().max() / ref.abs().max()) <= 2.0 ** -10
+
+
+# one row to past each tile's, columns in whole 16s and not (a multiple of 8 with zero-points),
+# K of one group, odd numbers of groups, past 16 and past 32 (the tables' chunks)
+@pytest.mark.parametrize("M,N,K", [(1, 1000, 128), (17, 136, 384), (33, 264, 2176), (49, 128, 4224),
+                                   (64, 520, 2048), (65, 1032, 4352), (129, 256, 6272), (200, 72, 12288)])
+@pytest.mark.parametrize("asym", [True, False])
+@pytest.mark.parametrize("kernel", ["prefill_wmma_ashuffle", "decode_gemv"])
+def test_few_tiles(M, N, K, asym, kernel):
+    _check(*_case(M, N, K, asym, M + N + K), kernel)
+
+
+# grids that take 64 x 128, 128 x 128 and 128 x 256 tiles (256 compute units), ragged at both ends
+@pytest.mark.parametrize("M,N,K", [(1090, 4104, 640), (1500, 8200, 384), (2050, 4360, 2304),
+                                   (1921, 16328, 256), (4097, 12296, 128)])
+@pytest.mark.parametrize("asym", [True, False])
+def test_many_tiles(M, N, K, asym):
+    _check(*_case(M, N, K, asym, M + N + K), "prefill_wmma_ashuffle")
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 256, 2048), (9, 512, 4096), (16, 256, 1024), (40, 1024, 2048),
+                                   (70, 520, 4352), (300, 1032, 1152)])
+def test_bf16_rows_equal_their_fp16_cast(M, N, K):
+    x, w, s, z = _case(M, N, K, True, M + K, torch.bfloat16)
+    args = (w, s, z, None, None, None, N, K, 128, True, 0, 0)
+    a = torch.ops.vllm.w4a8_dense_apply(x, *args)
+    b = torch.ops.vllm.w4a8_dense_apply(x.to(torch.float16), *args)
+    assert torch.equal(a, b)
