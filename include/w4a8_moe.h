@@ -302,6 +302,15 @@ W4A8_API int w4a8_moe_forward_noalloc(const void* x, int x_dtype, int64_t T, int
                                       int64_t num_global_experts, float* topk_weights,
                                       int32_t* topk_ids, void* out, void* stream);
 
+/* w4a8_mmq_fp8_gemm on int4 weights for fp16 or bf16 x (bf16 is cast to fp16 first, inside the
+ * kernels: the bits of a cast and the fp16 call): the dense linear layer behind
+ * vllm::w4a8_dense_apply (vllm_adapter.py:265-354). Workspace as w4a8_moe_gemm_workspace_size. */
+W4A8_API int w4a8_dense_linear(const void* x, int x_dtype, int64_t M, int64_t K,
+                               const int32_t* w_packed, const void* scales_f16,
+                               const int32_t* w_zeros, int64_t N, int64_t group_size,
+                               int64_t kernel, void* out_f16, void* workspace,
+                               size_t workspace_bytes, void* stream);
+
 /* Activations of w4a8_moe_mxfp4_apply. */
 #define W4A8_ACT_SILU 0        /* silu(gate) * up, w13 rows [gate | up] */
 #define W4A8_ACT_SWIGLUOAI 1   /* gpt-oss swigluoai, w13 rows interleaved (gate, up, gate, ...) */

@@ -120,6 +120,37 @@ int run_grouped(GroupedArgs& a, int64_t kernel, void* ws, size_t ws_bytes, hipSt
     return launch_grouped_scalar(a, s);
 }
 
+// The dense op: x (M, K) fp16 or bf16.
+int dense_impl(const void* x, bool x_bf16, int64_t M, int64_t K, const int32_t* w_packed,
+               const void* scales_f16, const int32_t* w_zeros, int64_t N, int64_t group_size,
+               int64_t kernel, int weight_is_e2m1, void* out_f16, void* workspace,
+               size_t workspace_bytes, hipStream_t s) {
+    W4A8_REQUIRE(M >= 0 && K > 0 && N > 0 && K % 8 == 0, "dense: invalid sizes");
+    W4A8_REQUIRE(group_size > 0 && K % group_size == 0, "K not divisible by scales' K dim");
+    W4A8_REQUIRE(group_size % 16 == 0 && group_size <= kMaxGroupSize,
+                 "group_size must be a multiple of 16 and <= 128");
+    W4A8_REQUIRE(dense_kernel_valid(kernel), "dense kernel id invalid (DenseKernel 0..14, no 3)");
+    W4A8_REQUIRE(!(weight_is_e2m1 && w_zeros), "mxfp4 (E2M1) weights are symmetric; w_zeros must be empty");
+    W4A8_REQUIRE(w_zeros == nullptr || N % 8 == 0, "w_zeros shape mismatch");
+    W4A8_REQUIRE(M == 0 || (x && w_packed && scales_f16 && out_f16), "dense: null pointer");
+    GroupedArgs a{};
+    a.x = x; a.x_bf16 = x_bf16; a.x_rows = M; a.K = K; a.w = w_packed;
+    a.scales = static_cast<const uint16_t*>(scales_f16); a.zeros = w_zeros;
+    a.E = 1; a.N = N; a.group_size = group_size;
+    a.sorted_ids = nullptr; a.P = M; a.expert_ids = nullptr; a.ntp = nullptr;
+    a.top_k = 1; a.identity_gather = false; a.num_valid = M;
+    a.e2m1 = weight_is_e2m1 != 0; a.epi = Epi::kHalf; a.out = out_f16; a.out_top_k = 1;
+    // DenseKernel 0 = reference_scalar, 11 = decode_gemv, everything else = matrix cores.
+    int64_t mk = W4A8_MOE_KERNEL_WMMA;
+    a.block_m = 64;
+    if (kernel == 0) { mk = W4A8_MOE_KERNEL_SCALAR; a.block_m = 1; }
+    if (kernel == 11) { mk = W4A8_MOE_KERNEL_GEMV; a.block_m = 16; }
+    // a few rows: the dense GEMV (rows quantised in the kernel, no act-quant launch)
+    if (kernel == 11 && dense_gemv_supported(M, N, K, group_size, weight_is_e2m1 != 0))
+        return launch_dense_gemv(x, x_bf16, M, K, w_packed, scales_f16, w_zeros, N, out_f16, s);
+    return run_grouped(a, mk, workspace, workspace_bytes, s);
+}
+
 }  // namespace
 
 void set_error(const std::string& msg) { g_error = msg; }
@@ -852,31 +883,18 @@ int w4a8_mmq_fp8_gemm(const void* x_f16, int64_t M, int64_t K, const int32_t* w_
                       int64_t group_size, int64_t kernel, int weight_is_e2m1, void* out_f16,
                       void* workspace, size_t workspace_bytes, void* stream) {
     clear_error();
-    W4A8_REQUIRE(M >= 0 && K > 0 && N > 0 && K % 8 == 0, "dense: invalid sizes");
-    W4A8_REQUIRE(group_size > 0 && K % group_size == 0, "K not divisible by scales' K dim");
-    W4A8_REQUIRE(group_size % 16 == 0 && group_size <= kMaxGroupSize,
-                 "group_size must be a multiple of 16 and <= 128");
-    W4A8_REQUIRE(dense_kernel_valid(kernel), "dense kernel id invalid (DenseKernel 0..14, no 3)");
-    W4A8_REQUIRE(!(weight_is_e2m1 && w_zeros), "mxfp4 (E2M1) weights are symmetric; w_zeros must be empty");
-    W4A8_REQUIRE(w_zeros == nullptr || N % 8 == 0, "w_zeros shape mismatch");
-    W4A8_REQUIRE(M == 0 || (x_f16 && w_packed && scales_f16 && out_f16), "dense: null pointer");
-    GroupedArgs a{};
-    a.x = x_f16; a.x_rows = M; a.K = K; a.w = w_packed;
-    a.scales = static_cast<const uint16_t*>(scales_f16); a.zeros = w_zeros;
-    a.E = 1; a.N = N; a.group_size = group_size;
-    a.sorted_ids = nullptr; a.P = M; a.expert_ids = nullptr; a.ntp = nullptr;
-    a.top_k = 1; a.identity_gather = false; a.num_valid = M;
-    a.e2m1 = weight_is_e2m1 != 0; a.epi = Epi::kHalf; a.out = out_f16; a.out_top_k = 1;
-    // DenseKernel 0 = reference_scalar, 11 = decode_gemv, everything else = matrix cores.
-    int64_t mk = W4A8_MOE_KERNEL_WMMA;
-    a.block_m = 64;
-    if (kernel == 0) { mk = W4A8_MOE_KERNEL_SCALAR; a.block_m = 1; }
-    if (kernel == 11) { mk = W4A8_MOE_KERNEL_GEMV; a.block_m = 16; }
-    // a few rows: the dense GEMV (rows quantised in the kernel, no act-quant launch)
-    if (kernel == 11 && dense_gemv_supported(M, N, K, group_size, weight_is_e2m1 != 0))
-        return launch_dense_gemv(x_f16, M, K, w_packed, scales_f16, w_zeros, N, out_f16,
-                                 as_stream(stream));
-    return run_grouped(a, mk, workspace, workspace_bytes, as_stream(stream));
+    return dense_impl(x_f16, false, M, K, w_packed, scales_f16, w_zeros, N, group_size, kernel,
+                      weight_is_e2m1, out_f16, workspace, workspace_bytes, as_stream(stream));
+}
+
+int w4a8_dense_linear(const void* x, int x_dtype, int64_t M, int64_t K, const int32_t* w_packed,
+                      const void* scales_f16, const int32_t* w_zeros, int64_t N,
+                      int64_t group_size, int64_t kernel, void* out_f16, void* workspace,
+                      size_t workspace_bytes, void* stream) {
+    clear_error();
+    W4A8_REQUIRE(x_dtype == W4A8_DTYPE_F16 || x_dtype == W4A8_DTYPE_BF16, "x dtype must be fp16 or bf16");
+    return dense_impl(x, x_dtype == W4A8_DTYPE_BF16, M, K, w_packed, scales_f16, w_zeros, N,
+                      group_size, kernel, 0, out_f16, workspace, workspace_bytes, as_stream(stream));
 }
 
 int w4a8_moe_apply_set_stage_events(void* const* events, int count) {

@@ -21,7 +21,7 @@ constexpr int kDgThreads = 64 * kDgWaves;
 constexpr uint32_t kDgOnes = 0x38383838u;   // four e4m3 bytes of 1.0
 
 struct DenseParams {
-    const __half* x;       // (M, K)
+    const uint16_t* x;     // (M, K) fp16 or bf16
     const int32_t* w;      // (N, K/8) op layout
     const __half* s;       // (N, G)
     const int32_t* z;      // (N/8, G) or null (uint4b8: zero point 8)
@@ -29,7 +29,14 @@ struct DenseParams {
     int M, N, K, G;
 };
 
-template <int GPW, bool ZP>
+// fp16 / bf16 bits -> f32; bf16 through fp16, the cast the reference applies first
+template <bool BF16>
+__device__ __forceinline__ float dg_f32(uint32_t bits) {
+    if constexpr (BF16) return __half2float(__float2half(__uint_as_float(bits << 16)));
+    return __half2float(__ushort_as_half((unsigned short)bits));
+}
+
+template <int GPW, bool ZP, bool BF16>
 __global__ void __launch_bounds__(kDgThreads) __attribute__((amdgpu_waves_per_eu(4))) dense_gemv_kernel(DenseParams p) {
     __shared__ float s_amax[kDgWaves][16];
     __shared__ v4f s_part[kDgWaves][64];
@@ -53,15 +60,16 @@ __global__ void __launch_bounds__(kDgThreads) __attribute__((amdgpu_waves_per_eu
     }
     // activation row c16 (pad rows repeat the last real row): k in [128 g + 32 q, +32)
     const int row = min(c16, p.M - 1);
-    const __half* xr = p.x + (int64_t)row * p.K + q * 32;
+    const uint16_t* xr = p.x + (int64_t)row * p.K + q * 32;
     uint4 raw[GPW][4];
 #pragma unroll
     for (int g = 0; g < GPW; ++g)
 #pragma unroll
         for (int i = 0; i < 4; ++i) raw[g][i] = *reinterpret_cast<const uint4*>(xr + (g0 + g) * kGroup + i * 8);
 
-    // row absmax on the magnitude bits (monotone in the fp16 value); a NaN, which fmaxf
-    // skips, lies above the infinity pattern and is dropped
+    // row absmax on the magnitude bits (both types are monotone in them, and so is the cast to
+    // fp16); a NaN, which fmaxf skips, lies above the infinity pattern and is dropped
+    constexpr uint32_t kInf = BF16 ? 0x7F80u : 0x7C00u;
     using u16x2 = unsigned short __attribute__((ext_vector_type(2)));
     u16x2 m2 = {0, 0};
 #pragma unroll
@@ -74,7 +82,7 @@ __global__ void __launch_bounds__(kDgThreads) __attribute__((amdgpu_waves_per_eu
                 m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2, wd[j] & 0x7FFF7FFFu));
         }
     uint32_t mbits = max((uint32_t)m2.x, (uint32_t)m2.y);
-    if (mbits > 0x7C00u) {
+    if (mbits > kInf) {
         mbits = 0;
 #pragma unroll
         for (int g = 0; g < GPW; ++g)
@@ -84,12 +92,12 @@ __global__ void __launch_bounds__(kDgThreads) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const uint32_t lo = wd[j] & 0x7FFFu, hi = (wd[j] >> 16) & 0x7FFFu;
-                    mbits = max(mbits, lo > 0x7C00u ? 0u : lo);
-                    mbits = max(mbits, hi > 0x7C00u ? 0u : hi);
+                    mbits = max(mbits, lo > kInf ? 0u : lo);
+                    mbits = max(mbits, hi > kInf ? 0u : hi);
                 }
             }
     }
-    float amax = __half2float(__ushort_as_half((unsigned short)mbits));
+    float amax = dg_f32<BF16>(mbits);
     {   // over the row's four quarter-lanes, then the eight waves' slices
         const auto r16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(amax), __float_as_uint(amax), false, false);
         amax = fmaxf(__uint_as_float(r16[0]), __uint_as_float(r16[1]));
@@ -111,8 +119,8 @@ __global__ void __launch_bounds__(kDgThreads) __attribute__((amdgpu_waves_per_eu
             float f[8];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                f[2 * j] = __half2float(__ushort_as_half((unsigned short)(wd[j] & 0xFFFFu))) * inv;
-                f[2 * j + 1] = __half2float(__ushort_as_half((unsigned short)(wd[j] >> 16))) * inv;
+                f[2 * j] = dg_f32<BF16>(wd[j] & 0xFFFFu) * inv;
+                f[2 * j + 1] = dg_f32<BF16>(wd[j] >> 16) * inv;
             }
             af[g][2 * i] = (int)pack4_e4m3(f[0], f[2], f[4], f[6]);
             af[g][2 * i + 1] = (int)pack4_e4m3(f[1], f[3], f[5], f[7]);
@@ -154,8 +162,10 @@ __global__ void __launch_bounds__(kDgThreads) __attribute__((amdgpu_waves_per_eu
 }
 
 template <int GPW, bool ZP>
-int launch_dense_t(const DenseParams& p, hipStream_t s) {
-    dense_gemv_kernel<GPW, ZP><<<dim3((unsigned)(p.N / 16)), dim3(kDgThreads), 0, s>>>(p);
+int launch_dense_t(const DenseParams& p, bool bf16, hipStream_t s) {
+    const dim3 grid((unsigned)(p.N / 16)), block(kDgThreads);
+    if (bf16) dense_gemv_kernel<GPW, ZP, true><<<grid, block, 0, s>>>(p);
+    else dense_gemv_kernel<GPW, ZP, false><<<grid, block, 0, s>>>(p);
     return check_launch("dense_gemv_kernel");
 }
 
@@ -167,14 +177,14 @@ bool dense_gemv_supported(int64_t M, int64_t N, int64_t K, int64_t group_size, b
            N * (K / 2) < ((int64_t)1 << 31);
 }
 
-int launch_dense_gemv(const void* x_f16, int64_t M, int64_t K, const int32_t* w, const void* scales_f16,
+int launch_dense_gemv(const void* x, bool x_bf16, int64_t M, int64_t K, const int32_t* w, const void* scales_f16,
                       const int32_t* zeros, int64_t N, void* out_f16, hipStream_t s) {
     if (!dense_gemv_supported(M, N, K, kGroup, false)) {
         set_error("dense GEMV: needs 1 <= M <= 16, group 128, K a multiple of 1024 up to 4096, N % 16 == 0");
         return W4A8_ERR_INVALID;
     }
     DenseParams p;
-    p.x = static_cast<const __half*>(x_f16);
+    p.x = static_cast<const uint16_t*>(x);
     p.w = w;
     p.s = static_cast<const __half*>(scales_f16);
     p.z = zeros;
@@ -186,10 +196,10 @@ int launch_dense_gemv(const void* x_f16, int64_t M, int64_t K, const int32_t* w,
     const int gpw = p.G / kDgWaves;
     const bool zp = zeros != nullptr;
     switch (gpw) {
-        case 1: return zp ? launch_dense_t<1, true>(p, s) : launch_dense_t<1, false>(p, s);
-        case 2: return zp ? launch_dense_t<2, true>(p, s) : launch_dense_t<2, false>(p, s);
-        case 3: return zp ? launch_dense_t<3, true>(p, s) : launch_dense_t<3, false>(p, s);
-        default: return zp ? launch_dense_t<4, true>(p, s) : launch_dense_t<4, false>(p, s);
+        case 1: return zp ? launch_dense_t<1, true>(p, x_bf16, s) : launch_dense_t<1, false>(p, x_bf16, s);
+        case 2: return zp ? launch_dense_t<2, true>(p, x_bf16, s) : launch_dense_t<2, false>(p, x_bf16, s);
+        case 3: return zp ? launch_dense_t<3, true>(p, x_bf16, s) : launch_dense_t<3, false>(p, x_bf16, s);
+        default: return zp ? launch_dense_t<4, true>(p, x_bf16, s) : launch_dense_t<4, false>(p, x_bf16, s);
     }
 }
 

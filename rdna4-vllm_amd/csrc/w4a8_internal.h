@@ -177,10 +177,10 @@ struct GroupedArgs {
     float alpha, limit;
 };
 
-// Dense GEMV for 1 <= M <= 16 rows of fp16 x on op-layout weights (dense_gemv.hip): group
+// Dense GEMV for 1 <= M <= 16 rows of fp16 or bf16 x on op-layout weights (dense_gemv.hip): group
 // 128, K a multiple of 1024 up to 4096, N % 16 == 0; quantises the rows itself.
 bool dense_gemv_supported(int64_t M, int64_t N, int64_t K, int64_t group_size, bool e2m1);
-int launch_dense_gemv(const void* x_f16, int64_t M, int64_t K, const int32_t* w, const void* scales_f16,
+int launch_dense_gemv(const void* x, bool x_bf16, int64_t M, int64_t K, const int32_t* w, const void* scales_f16,
                       const int32_t* zeros, int64_t N, void* out_f16, hipStream_t s);
 // Wide streamed-K tiles (wide_tiles.hip): op-layout int4 weights of group 128, any K, rows
 // prequantised with group sums, fp16 out.

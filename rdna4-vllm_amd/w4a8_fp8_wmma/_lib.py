@@ -51,6 +51,8 @@ SIGNATURES = {
                                       _c_void_p, _c_void_p]),
     "w4a8_mmq_fp8_gemm": (_int, [_c_void_p, _i64, _i64, _c_void_p, _c_void_p, _c_void_p, _i64,
                                  _i64, _i64, _int, _c_void_p, _c_void_p, _size, _c_void_p]),
+    "w4a8_dense_linear": (_int, [_c_void_p, _int, _i64, _i64, _c_void_p, _c_void_p, _c_void_p,
+                                 _i64, _i64, _i64, _c_void_p, _c_void_p, _size, _c_void_p]),
     "w4a8_moe_apply_workspace_size": (_size, [_i64, _i64, _i64, _i64, _i64]),
     "w4a8_moe_apply_set_stage_events": (_int, [ctypes.POINTER(_c_void_p), _int]),
     "w4a8_moe_apply": (_int, [_c_void_p, _int, _i64, _i64, _i64, _i64, _i64, _i64, _c_void_p,

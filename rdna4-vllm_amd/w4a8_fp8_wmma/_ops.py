@@ -190,10 +190,9 @@ def mmq_fp8_moe_gather_reduce_cuda(out2, sorted_token_ids, topk_weights,
     return out
 
 
-def mmq_fp8_gemm_cuda(x, w_packed, scales, w_zeros, kernel, weight_is_e2m1=False):
-    """bindings.cpp:98-146."""
+def _check_dense(x, w_packed, scales, w_zeros, weight_is_e2m1):
+    """The dense op's tensors (bindings.cpp:98-121), x's dtype aside: (M, N, K, group, zeros)."""
     _check(x.is_cuda and w_packed.is_cuda and scales.is_cuda, "x, w_packed, scales must be CUDA")
-    _check(x.dtype == torch.float16, "x must be fp16")
     _check(w_packed.dtype == torch.int32, "w_packed must be int32")
     _check(scales.dtype == torch.float16, "scales must be fp16")
     _check(x.dim() == 2 and w_packed.dim() == 2 and scales.dim() == 2, "all inputs must be 2D")
@@ -205,8 +204,26 @@ def mmq_fp8_gemm_cuda(x, w_packed, scales, w_zeros, kernel, weight_is_e2m1=False
            f"w_packed last dim mismatch: expected K/8 = {K // 8} got {w_packed.size(1)}")
     _check(scales.size(0) == N, f"scales.size(0) must equal N={N}")
     _check(scales.size(1) > 0 and K % scales.size(1) == 0, "K not divisible by scales' K dim")
-    gs = K // scales.size(1)
-    z = _zeros_or_none(w_zeros, N, scales, weight_is_e2m1, 2)
+    return M, N, K, K // scales.size(1), _zeros_or_none(w_zeros, N, scales, weight_is_e2m1, 2)
+
+
+def dense_linear(x, w_packed, scales, w_zeros, kernel):
+    """The dense op on int4 weights for fp16 or bf16 x: the bits of mmq_fp8_gemm on x cast to
+    fp16, without the cast's launch. kernel: dense op id."""
+    _check(x.dtype in (torch.float16, torch.bfloat16), "x must be fp16 or bf16")
+    M, N, K, gs, z = _check_dense(x, w_packed, scales, w_zeros, False)
+    out = torch.empty((M, N), dtype=torch.float16, device=x.device)
+    ws = _workspace(lib.w4a8_moe_gemm_workspace_size(M, K), x.device)
+    check(lib.w4a8_dense_linear(
+        _ptr(x), 1 if x.dtype == torch.bfloat16 else 0, M, K, _ptr(w_packed), _ptr(scales), _ptr(z),
+        N, gs, kernel, _ptr(out), ws.data_ptr(), ws.numel(), _stream(x)), "dense_linear")
+    return out
+
+
+def mmq_fp8_gemm_cuda(x, w_packed, scales, w_zeros, kernel, weight_is_e2m1=False):
+    """bindings.cpp:98-146."""
+    _check(x.dtype == torch.float16, "x must be fp16")
+    M, N, K, gs, z = _check_dense(x, w_packed, scales, w_zeros, weight_is_e2m1)
     out = torch.empty((M, N), dtype=torch.float16, device=x.device)
     ws = _workspace(lib.w4a8_moe_gemm_workspace_size(M, K), x.device)
     check(lib.w4a8_mmq_fp8_gemm(

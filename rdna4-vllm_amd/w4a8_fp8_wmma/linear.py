@@ -28,7 +28,8 @@ from typing import Optional
 
 import torch
 
-from . import mmq_fp8_gemm
+from . import _DENSE_KERNELS, mmq_fp8_gemm
+from ._ops import dense_linear
 
 logger = logging.getLogger(__name__)
 
@@ -74,12 +75,9 @@ def dense_kernel_for(M: int, N: int, K: int, group_size: int) -> str:
     return "prefill_wmma_ashuffle" if group_size in (32, 128) else "prefill_wmma"
 
 
-def w4a8_dense_apply(x2d: torch.Tensor, w_q: torch.Tensor, w_s: torch.Tensor,
-                     w_zp: Optional[torch.Tensor], tri_bq: Optional[torch.Tensor],
-                     tri_s: Optional[torch.Tensor], tri_zp: Optional[torch.Tensor],
-                     N: int, K: int, group_size: int, zero_points: bool,
-                     weight_type_bias: int, cached_min_m: int) -> torch.Tensor:
-    """One dense W4A8 linear: x2d (M, K) -> (M, N) fp16 (vllm_adapter.py:265-354)."""
+def _dense_args(x2d, w_q, w_s, w_zp, tri_bq, tri_s, tri_zp, N, K, group_size, zero_points,
+                weight_type_bias, cached_min_m):
+    """The op's checks: (x2d, weights, scales, zero points or None, kernel name)."""
     del tri_bq, tri_s, tri_zp, cached_min_m   # Triton fallback inputs: no Triton here
     if _force_mode() == "off":
         raise RuntimeError("VLLM_ROCM_W4A8_FORCE=off selects the stock Triton path, which "
@@ -92,11 +90,27 @@ def w4a8_dense_apply(x2d: torch.Tensor, w_q: torch.Tensor, w_s: torch.Tensor,
     if not use_zp and int(weight_type_bias) != UINT4B8_BIAS:
         raise ValueError("weights without zero points must be uint4b8 (bias 8), "
                          f"got bias {weight_type_bias}")
-    if x2d.dtype != torch.float16:
-        x2d = x2d.to(torch.float16)
-    x2d = x2d.contiguous()
-    kernel = dense_kernel_for(x2d.shape[0], N, K, group_size)
-    return mmq_fp8_gemm(x2d, w_q, w_s, kernel=kernel, w_zeros=w_zp if use_zp else None)
+    return x2d, w_q, w_s, w_zp if use_zp else None, dense_kernel_for(x2d.shape[0], N, K, group_size)
+
+
+def w4a8_dense_apply(x2d: torch.Tensor, w_q: torch.Tensor, w_s: torch.Tensor,
+                     w_zp: Optional[torch.Tensor], tri_bq: Optional[torch.Tensor],
+                     tri_s: Optional[torch.Tensor], tri_zp: Optional[torch.Tensor],
+                     N: int, K: int, group_size: int, zero_points: bool,
+                     weight_type_bias: int, cached_min_m: int) -> torch.Tensor:
+    """One dense W4A8 linear: x2d (M, K) -> (M, N) fp16 (vllm_adapter.py:265-354)."""
+    x, w, s, z, kernel = _dense_args(x2d, w_q, w_s, w_zp, tri_bq, tri_s, tri_zp, N, K, group_size,
+                                     zero_points, weight_type_bias, cached_min_m)
+    return mmq_fp8_gemm(x.to(torch.float16).contiguous(), w, s, kernel=kernel, w_zeros=z)
+
+
+def _w4a8_dense_apply_cuda(*args) -> torch.Tensor:
+    """The op's CUDA(HIP) kernel: below the dispatcher, so straight to the C ABI; bf16 rows are
+    cast inside the kernels (the same bits, one launch less)."""
+    x, w, s, z, kernel = _dense_args(*args)
+    if x.dtype not in (torch.float16, torch.bfloat16):
+        x = x.to(torch.float16)
+    return dense_linear(x.contiguous(), w, s, z, _DENSE_KERNELS[kernel])
 
 
 def _w4a8_dense_apply_fake(x2d, w_q, w_s, w_zp, tri_bq, tri_s, tri_zp, N, K, group_size,
@@ -118,7 +132,7 @@ def register_dense_op() -> None:
         return
     lib = torch.library.Library("vllm", "FRAGMENT")
     lib.define(_SCHEMA)
-    lib.impl("w4a8_dense_apply", w4a8_dense_apply, "CUDA")
+    lib.impl("w4a8_dense_apply", _w4a8_dense_apply_cuda, "CUDA")
     torch.library.register_fake("vllm::w4a8_dense_apply", _w4a8_dense_apply_fake, lib=lib)
     _vllm_lib = lib
 
