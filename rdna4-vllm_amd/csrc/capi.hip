@@ -70,7 +70,9 @@ int run_grouped(GroupedArgs& a, int64_t kernel, void* ws, size_t ws_bytes, hipSt
     a.act_scales = w.take<float>((size_t)a.x_rows);
     float* gsum = w.take<float>((size_t)(a.x_rows * ((a.K + 127) / 128)));
     const bool have_ws = !(a.x_rows > 0 && ws == nullptr) && w.ok();
-    if (dense && have_ws && (a.P + 15) / 16 * a.N > 16 * 1024) gemv = false;
+    const bool whole = gemv_whole_split(a.K, a.group_size);
+    if (dense && have_ws && (!whole || (a.P + 15) / 16 * a.N > 16 * 1024)) gemv = false;
+    if (!have_ws && !whole) gemv = false;   // uneven groups take quantised rows (refused below)
     // identity-gathered inputs (gemm2 / scatter) have one row per padded row: skip padding.
     const bool filter = a.identity_gather && a.sorted_ids != nullptr;
     if (kernel == W4A8_MOE_KERNEL_GEMV && gemv) {
@@ -347,7 +349,7 @@ inline void stamp_gemm(int gemm) {
 // Fragment-layout weights are read by the decode GEMV and the prefill tiles only.
 bool fragments_schedule_ok(bool decode, int64_t H, int64_t inter, int64_t gs) {
     if (gs != 128 || H % 128 != 0 || inter % 128 != 0) return false;
-    if (decode) return gemv_supported(H, gs) && gemv_supported(inter, gs);
+    if (decode) return gemv_whole_split(H, gs) && gemv_whole_split(inter, gs);
     return prefill_supported(H, gs, false) && prefill_supported(inter, gs, false);
 }
 

@@ -390,19 +390,32 @@ constexpr int kGemvMaxRows = 64;                 // block_m cap (16-row passes)
 constexpr int kGemvMaxTiles = 8;                 // tiles per team (LDS partials bound)
 constexpr uint32_t kOnesE4m3 = 0x38383838u;      // four e4m3 bytes of 1.0
 
-template <Epi EPI, int GPW, int KSPLIT>
+// RAG: the waves' GPW groups together pass K's. The missing groups of the last waves read the
+// last group again and count with scale 0. A row's scales and zero-points start at any 2 (4)
+// bytes, so a lane could only load them one by one; the work-group puts those of all its
+// columns into an LDS table instead (E = 128, top-8, hidden 2304, intermediate 896, T = 24, the
+// two GEMVs on raw nibbles: 47.3 + 25.4 us, 56.4 + 31.6 with single loads beside the weights).
+// The nibbles enter the MFMA decoded to e4m3(n - z), as in the tiles that ran these sizes before:
+// raw ones leave four times the rounding in the partial sums (8 instead of 2 in 100 fp16
+// results off by an ulp). The decode's VALU makes it 56.7 + 30.5 us (3.6 and 3.4 TB/s).
+template <Epi EPI, int GPW, int KSPLIT, bool RAG = false>
 struct GemvCfg {
     static constexpr bool kSilu = EPI == Epi::kSiluHalf;
     static constexpr int NF = kSilu ? 2 : 1;      // fragments per column tile
     static constexpr int CT = kSilu ? 1 : 2;      // column tiles per chunk
     static constexpr int FR = NF * CT;            // fragments per chunk and group
-    static constexpr int GC = GPW < 4 ? GPW : 4;  // groups per chunk
+    static constexpr int GC = GPW < 4 || GPW == 5 ? GPW : GPW == 6 ? 3 : 4;  // groups per chunk
     static constexpr int NB = GPW / GC;           // chunks per tile set
     static constexpr int TEAMS = 4 / KSPLIT;      // wave teams (independent tile ranges)
-    static constexpr bool kPackedScales = GC == 2 || GC == 4;
     // 4-group chunks (one per tile set): the scales and zero-point words of all chunks are
     // loaded once per work-group into LDS instead of alongside every chunk
-    static constexpr bool kStagedSZ = GC == 4 && NB == 1;
+    static constexpr bool kStagedSZ = GC == 4 && NB == 1 && !RAG;
+    // RAG: one word per column and group (fp16 scale, zero-point << 16), an odd row stride
+    static constexpr int GP = GPW * KSPLIT;
+    static constexpr int kTabRow = GP | 1;
+    static constexpr int kTabCols = TEAMS * kGemvMaxTiles * 16;
+    static constexpr int kTabWords = RAG ? NF * kTabCols * kTabRow : 1;
+    static constexpr int kTabItems = RAG ? (NF * kTabCols / 8 * GP + 255) / 256 : 1;
     static_assert(GPW % GC == 0 && (NB == 1 || NB == 2), "unsupported groups per wave");
     static_assert(KSPLIT == 1 || KSPLIT == 2 || KSPLIT == 4, "KSPLIT divides the 4 waves");
 };
@@ -471,9 +484,10 @@ __device__ __forceinline__ float act_bits_to_f32(uint32_t bits, bool bf16) {
 // act_quant_kernel (the row absmax is combined across the KSPLIT waves through LDS).
 // FRAG: weights in the fragment layout (repack.hip): a fragment-group is one contiguous
 // kilobyte, lane l's 16 bytes at offset 16 l.
-template <Epi EPI, int GPW, int KSPLIT, bool AQ, bool FRAG>
+template <Epi EPI, int GPW, int KSPLIT, bool AQ, bool FRAG, bool RAG = false>
 __global__ void __launch_bounds__(256, 2) grouped_gemv_kernel(Params p, int tpt) {
-    using C = GemvCfg<EPI, GPW, KSPLIT>;
+    using C = GemvCfg<EPI, GPW, KSPLIT, RAG>;
+    static_assert(!RAG || (!AQ && !FRAG), "ragged groups: prequantised rows, op layout");
     extern __shared__ __attribute__((aligned(16))) uint8_t s_dyn[];   // KSPLIT > 1 partials
     __shared__ float s_amax[4][16];
     __shared__ int s_opad[4][16];
@@ -483,6 +497,8 @@ __global__ void __launch_bounds__(256, 2) grouped_gemv_kernel(Params p, int tpt)
     // chunk of the wave: [chunk][fragment][column] and [chunk][fragment][column / 8]
     __shared__ uint2 s_sc[4][C::kStagedSZ ? kGemvMaxTiles * C::FR * 16 : 1];
     __shared__ uint4 s_zw[4][C::kStagedSZ ? kGemvMaxTiles * C::FR * 2 : 1];
+    __shared__ uint32_t s_tab[C::kTabWords];   // [gate | up][column][kTabRow]
+    __shared__ uint4 s_lut[RAG ? 16 : 1];      // e4m3(n - z) tables
     v4f* s_part = reinterpret_cast<v4f*>(s_dyn);   // [wave][tile][NF][lane]
 
     const int tid = threadIdx.x;
@@ -542,13 +558,15 @@ __global__ void __launch_bounds__(256, 2) grouped_gemv_kernel(Params p, int tpt)
     // for everything at the join). Word u * FR + f of a chunk = group u, fragment f,
     // quarter q of this lane's column.
     uint4 wv[2][C::GC * C::FR];
-    uint32_t sw[2][C::kStagedSZ ? 1 : C::FR][C::GC];
-    int32_t zw[2][C::kStagedSZ ? 1 : C::FR][C::GC];
+    constexpr bool kWithChunk = !C::kStagedSZ && !RAG;   // scales loaded beside each chunk
+    uint32_t sw[2][kWithChunk ? C::FR : 1][C::GC];
+    int32_t zw[2][kWithChunk ? C::FR : 1][C::GC];
     auto issue = [&](int c, auto bufc) {
         constexpr int b = decltype(bufc)::value;
         const bool live = c < nch;
         const int t = t_begin + (c / C::NB) * C::CT;
-        const int g = live ? g0 + (c % C::NB) * C::GC : g0;
+        const int gr = live ? g0 + (c % C::NB) * C::GC : g0;
+        const int g = RAG ? min(gr, p.G - 1) : gr;
         // byte offsets: a wave-uniform part (group, step) on a scalar base plus a 32-bit lane
         // part (the expert's slice is < 2^31 bytes); past the end every lane reads offset 0
         constexpr uint32_t ustep = FRAG ? 1024u : kGroup / 2;
@@ -566,10 +584,11 @@ __global__ void __launch_bounds__(256, 2) grouped_gemv_kernel(Params p, int tpt)
             // next instruction reads, so they stay cached
 #pragma unroll
             for (int u = 0; u < C::GC; ++u) {
-                const uint8_t* ptr = wg + (live ? u * ustep : 0u) + opaque_u32(woff);
+                const uint32_t uo = RAG ? (uint32_t)min(u, p.G - 1 - g) : (uint32_t)u;   // g <= G - 1
+                const uint8_t* ptr = wg + (live ? uo * ustep : 0u) + opaque_u32(woff);
                 wv[b][u * C::FR + f] = FRAG ? load_stream16(ptr) : *reinterpret_cast<const uint4*>(ptr);
             }
-            if constexpr (!C::kStagedSZ) {
+            if constexpr (kWithChunk) {
                 load_scales<C::GC>(reinterpret_cast<const __half*>(
                                        reinterpret_cast<const uint8_t*>(se) + (uint32_t)g * 2u +
                                        opaque_u32((uint32_t)n * (uint32_t)p.G * 2u)),
@@ -610,6 +629,30 @@ __global__ void __launch_bounds__(256, 2) grouped_gemv_kernel(Params p, int tpt)
         }
     }
 
+    // ---- level 2a (ragged groups): the work-group's table, a thread eight columns of a group ----
+    const int tab_cb = blockIdx.x * C::TEAMS * tpt * 2;       // first block of 8 columns
+    const int tab_nb = C::TEAMS * tpt * 2;                    // blocks, of gate and of up each
+    const int tab_items = C::NF * tab_nb * C::GP;             // <= 256 * kTabItems
+    uint16_t ts[C::kTabItems][8];
+    int32_t tz[C::kTabItems][2];
+    if constexpr (RAG) {
+#pragma unroll
+        for (int i = 0; i < C::kTabItems; ++i) {
+            const int it = min(i * 256 + tid, tab_items - 1);
+            const int blk = it / C::GP;
+            const uint32_t gg = (uint32_t)min(it % C::GP, p.G - 1);
+            const bool up = blk >= tab_nb;
+            const int n0 = (tab_cb + (up ? blk - tab_nb : blk)) * 8 + (up ? ncols : 0);
+#pragma unroll
+            for (int j = 0; j < 8; ++j)   // rows past the end: their columns are never stored
+                ts[i][j] = reinterpret_cast<const uint16_t*>(se)[(uint32_t)min(n0 + j, p.N - 1) * (uint32_t)p.G + gg];
+            // up may start inside a word of eight zero-points: the eight lie in two words
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                tz[i][j] = ze ? ze[(uint32_t)(min(n0 + 7 * j, p.N - 1) >> 3) * (uint32_t)p.G + gg] : 0;
+        }
+    }
+
     for (int m0 = 0; m0 < mreal; m0 += 16) {
         if (m0 > 0) __syncthreads();   // LDS partials / row maxima of the previous pass consumed
         // A row m0 + c16 of this pass (pad rows repeat the last real row)
@@ -622,8 +665,9 @@ __global__ void __launch_bounds__(256, 2) grouped_gemv_kernel(Params p, int tpt)
             const uint8_t* xr = p.xq + (int64_t)asrc * p.K + q * 32;
 #pragma unroll
             for (int u = 0; u < GPW; ++u) {
-                const uint4 lo = *reinterpret_cast<const uint4*>(xr + (g0 + u) * kGroup);
-                const uint4 hi = *reinterpret_cast<const uint4*>(xr + (g0 + u) * kGroup + 16);
+                const int gu = RAG ? min(g0 + u, p.G - 1) : g0 + u;
+                const uint4 lo = *reinterpret_cast<const uint4*>(xr + gu * kGroup);
+                const uint4 hi = *reinterpret_cast<const uint4*>(xr + gu * kGroup + 16);
                 af[u] = v8i{(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w,
                             (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
             }
@@ -705,7 +749,7 @@ __global__ void __launch_bounds__(256, 2) grouped_gemv_kernel(Params p, int tpt)
         }
         v4f sa[GPW];   // 2^-9 * group sums of rows 4q..4q+3
 #pragma unroll
-        for (int u = 0; u < GPW; ++u) {
+        for (int u = 0; u < (RAG ? 0 : GPW); ++u) {
             const int one = (int)kOnesE4m3;
             sa[u] = mfma_16x16x128(af[u], v8i{one, one, one, one, one, one, one, one},
                                    v4f{0.f, 0.f, 0.f, 0.f});
@@ -721,12 +765,34 @@ __global__ void __launch_bounds__(256, 2) grouped_gemv_kernel(Params p, int tpt)
             }
         }
 
+        if constexpr (RAG) {
+            if (m0 == 0) {
+#pragma unroll
+                for (int i = 0; i < C::kTabItems; ++i) {
+                    const int it = min(i * 256 + tid, tab_items - 1);
+                    const int blk = it / C::GP, gt = it % C::GP;
+                    const bool up = blk >= tab_nb;
+                    const int n0 = (tab_cb + (up ? blk - tab_nb : blk)) * 8 + (up ? ncols : 0);
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) {
+                        const int n = n0 + j;
+                        const int z = ze ? ((n >> 3) == (n0 >> 3) ? tz[i][0] : tz[i][1]) >> ((n & 7) * 4) & 0xF : 8;
+                        const uint32_t sc = gt < p.G ? ts[i][j] : 0u;
+                        s_tab[(blk * 8 + j) * C::kTabRow + gt] =
+                            sc | (uint32_t)z << 16;
+                    }
+                }
+                if (tid < 16) s_lut[tid] = load_table(tid);
+                lds_barrier();
+            }
+        }
+
         // per-wave table of this pass's 16 output rows (padded row, slot, scale), read back
         // at store time instead of being held in registers across the chunk loop
         if (q == 0) {
             const int j = nth_set_bit(vmask, min(m0 + c16, mreal - 1));
             s_opad[wave][c16] = (int)(row0 + j);
-            s_oasc[wave][c16] = my_asc * wscale;
+            s_oasc[wave][c16] = RAG ? my_asc : my_asc * wscale;
         }
         {
             const int j = nth_set_bit(vmask, min(m0 + c16, mreal - 1));
@@ -761,7 +827,10 @@ __global__ void __launch_bounds__(256, 2) grouped_gemv_kernel(Params p, int tpt)
             const int t = t_begin + (c / C::NB) * C::CT;
 #pragma unroll
             for (int f = 0; f < C::FR; ++f) {
-                const int zsh = (row_of(t, f) & 7) * 4;
+                const int zsh = RAG ? 0 : (row_of(t, f) & 7) * 4;
+                // (a tile past the wave's last one reads that one's words: never stored)
+                const int tabc = ((C::kSilu && f >= C::CT ? tab_nb / 2 : 0) +
+                                  min(t + f % C::CT, t_begin + tpt - 1) - tab_cb / 2) * 16 + c16;
                 uint32_t scw[C::GC];
                 int32_t zwd[C::GC];
                 if constexpr (C::kStagedSZ) {
@@ -773,7 +842,7 @@ __global__ void __launch_bounds__(256, 2) grouped_gemv_kernel(Params p, int tpt)
                     zwd[1] = (int32_t)zv.y;
                     zwd[2] = (int32_t)zv.z;
                     zwd[3] = (int32_t)zv.w;
-                } else {
+                } else if constexpr (!RAG) {
 #pragma unroll
                     for (int u = 0; u < C::GC; ++u) {
                         scw[u] = sw[b][f][u];
@@ -783,12 +852,21 @@ __global__ void __launch_bounds__(256, 2) grouped_gemv_kernel(Params p, int tpt)
 #pragma unroll
                 for (int u = 0; u < C::GC; ++u) {
                     const int ua = gb * C::GC + u;
-                    v4f acc = mfma_16x16x128(af[ua], spread_nibbles(wv[b][u * C::FR + f]),
+                    v4f acc;
+                    float s;
+                    if constexpr (RAG) {
+                        const uint32_t tw = s_tab[tabc * C::kTabRow + g0 + ua];
+                        s = __half2float(__ushort_as_half((unsigned short)tw));
+                        acc = mfma_16x16x128(af[ua], decode_frag(wv[b][u * C::FR + f], s_lut[tw >> 16]),
                                              v4f{0.f, 0.f, 0.f, 0.f});
-                    const float z = ze ? (float)((zwd[u] >> zsh) & 0xF) : 8.0f;
+                    } else {
+                        acc = mfma_16x16x128(af[ua], spread_nibbles(wv[b][u * C::FR + f]),
+                                             v4f{0.f, 0.f, 0.f, 0.f});
+                        const float z = ze ? (float)((zwd[u] >> zsh) & 0xF) : 8.0f;
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[r] = fmaf(-z, sa[ua][r], acc[r]);
-                    const float s = scale_at<C::GC>(scw, u);
+                        for (int r = 0; r < 4; ++r) acc[r] = fmaf(-z, sa[ua][r], acc[r]);
+                        s = scale_at<C::GC>(scw, u);
+                    }
 #pragma unroll
                     for (int r = 0; r < 4; ++r) run[f][r] = fmaf(acc[r], s, run[f][r]);
                 }
@@ -901,12 +979,21 @@ int launch_mfma_e(const Params& p, hipStream_t s) {
     return launch_mfma_b<EPI>(p, s);
 }
 
-// Split of the K groups over waves: G == GPW * KSPLIT for the shapes below; others run
-// the matrix-core tiles.
+// Split of the K groups over waves: G == GPW * KSPLIT for the shapes below; others up to 32
+// take the next larger split with the last wave's missing groups masked (ragged), and past that
+// the matrix-core tiles. E = 128, top-8, hidden 2304 (18 groups), intermediate 896 (7), T = 24,
+// the layer: 140 us on the tiles (87.6 + 43.4), 95 here; T = 1 44 / 41, T = 96 185 / 120.
 struct GemvSplit {
     int gpw, ksplit;
+    bool ragged = false;
 };
 GemvSplit gemv_split(int G) {
+    if (G == 5) return {3, 2, true};
+    if (G == 7) return {4, 2, true};
+    if (G >= 9 && G <= 11) return {3, 4, true};
+    if (G >= 13 && G <= 15) return {4, 4, true};
+    if (G >= 17 && G <= 20) return {5, 4, true};
+    if (G >= 21 && G <= 24) return {6, 4, true};
     switch (G) {
         case 1: return {1, 1};
         case 2: return {2, 1};
@@ -923,37 +1010,46 @@ GemvSplit gemv_split(int G) {
 
 // Column tiles per wave team: enough work per work-group to hide the prologue (~64 KB of
 // weights per wave), fewer when the grid would otherwise leave CUs idle (two work-groups
-// per CU fit; 512 keeps every CU of a 256-CU part busy).
-int gemv_default_tpt(const Params& p, int ntiles, int frag_bytes_per_tile_wave, int teams) {
+// per CU fit; 512 keeps every CU of a 256-CU part busy). Ragged groups decode their weights, so
+// a second round that is nearly empty costs more: from 384 (E = 128, hidden 2304, T = 3: 41 us a
+// layer, 51 from 512, 58 from 1024; T = 1, 2 and 4 to 24 within 3% of the best).
+int gemv_default_tpt(const Params& p, int ntiles, int frag_bytes_per_tile_wave, int teams, int min_wgs) {
     const int64_t blocks = std::min<int64_t>((p.P + p.block_m - 1) / p.block_m, p.num_valid);
     int tpt = std::max(1, (64 * 1024) / frag_bytes_per_tile_wave);
     tpt = std::min(tpt, kGemvMaxTiles);
-    // keep >= ~512 work-groups when the routing touches few blocks (T = 1 decode)
-    while (tpt > 1 && blocks * ((ntiles + teams * tpt - 1) / (teams * tpt)) < 512) tpt >>= 1;
+    // keep >= min_wgs work-groups when the routing touches few blocks (T = 1 decode)
+    while (tpt > 1 && blocks * ((ntiles + teams * tpt - 1) / (teams * tpt)) < min_wgs) tpt >>= 1;
     return tpt;
 }
 
-template <Epi EPI, int GPW, int KSPLIT, bool AQ, bool FRAG>
+template <Epi EPI, int GPW, int KSPLIT, bool AQ, bool FRAG, bool RAG = false>
 int launch_gemv_a(const Params& p, int tpt, dim3 grid, size_t lds, hipStream_t s) {
-    using C = GemvCfg<EPI, GPW, KSPLIT>;
-    if (int rc = reserve_dyn_lds(reinterpret_cast<const void*>(&grouped_gemv_kernel<EPI, GPW, KSPLIT, AQ, FRAG>),
+    using C = GemvCfg<EPI, GPW, KSPLIT, RAG>;
+    if (int rc = reserve_dyn_lds(reinterpret_cast<const void*>(&grouped_gemv_kernel<EPI, GPW, KSPLIT, AQ, FRAG, RAG>),
                                  4 * kGemvMaxTiles * C::NF * 64 * (int)sizeof(v4f),
                                  "grouped_gemv_kernel"))
         return rc;
-    launch_kernel(&grouped_gemv_kernel<EPI, GPW, KSPLIT, AQ, FRAG>, grid, dim3(256), lds, s, p, tpt);
+    launch_kernel(&grouped_gemv_kernel<EPI, GPW, KSPLIT, AQ, FRAG, RAG>, grid, dim3(256), lds, s, p, tpt);
     return check_launch("grouped_gemv_kernel");
 }
 
-template <Epi EPI, int GPW, int KSPLIT>
+template <Epi EPI, int GPW, int KSPLIT, bool RAG = false>
 int launch_gemv_t(const Params& p, int tpt, hipStream_t s) {
-    using C = GemvCfg<EPI, GPW, KSPLIT>;
+    using C = GemvCfg<EPI, GPW, KSPLIT, RAG>;
     const int ncols = C::kSilu ? p.N / 2 : p.N;
     const int ntiles = (ncols + 15) / 16;
-    if (tpt <= 0) tpt = gemv_default_tpt(p, ntiles, GPW * C::NF * 1024, C::TEAMS);
+    if (tpt <= 0) tpt = gemv_default_tpt(p, ntiles, GPW * C::NF * 1024, C::TEAMS, RAG ? 384 : 512);
     tpt = std::min(tpt, kGemvMaxTiles);
     const size_t lds = KSPLIT > 1 ? (size_t)4 * tpt * C::NF * 64 * sizeof(v4f) : 0;
     const dim3 grid((unsigned)((ntiles + C::TEAMS * tpt - 1) / (C::TEAMS * tpt)),
                     (unsigned)((p.P + p.block_m - 1) / p.block_m));
+    if constexpr (RAG) {
+        if (!p.xq || p.w_frag) {
+            set_error("grouped GEMV: this number of K groups needs prequantised rows and op-layout weights");
+            return W4A8_ERR_INVALID;
+        }
+        return launch_gemv_a<EPI, GPW, KSPLIT, false, false, true>(p, tpt, grid, lds, s);
+    } else {
     if (p.w_frag) {
         // fragment-layout weights come only with prequantised rows (the whole-layer path)
         if (!p.xq) {
@@ -964,11 +1060,22 @@ int launch_gemv_t(const Params& p, int tpt, hipStream_t s) {
     }
     if (p.xq) return launch_gemv_a<EPI, GPW, KSPLIT, false, false>(p, tpt, grid, lds, s);
     return launch_gemv_a<EPI, GPW, KSPLIT, true, false>(p, tpt, grid, lds, s);
+    }
 }
 
 template <Epi EPI>
 int launch_gemv_e(const Params& p, int tpt, hipStream_t s) {
     const GemvSplit sp = gemv_split(p.G);
+    if (sp.ragged) {
+        switch (sp.gpw * 8 + sp.ksplit) {
+            case 3 * 8 + 2: return launch_gemv_t<EPI, 3, 2, true>(p, tpt, s);
+            case 4 * 8 + 2: return launch_gemv_t<EPI, 4, 2, true>(p, tpt, s);
+            case 3 * 8 + 4: return launch_gemv_t<EPI, 3, 4, true>(p, tpt, s);
+            case 4 * 8 + 4: return launch_gemv_t<EPI, 4, 4, true>(p, tpt, s);
+            case 5 * 8 + 4: return launch_gemv_t<EPI, 5, 4, true>(p, tpt, s);
+            case 6 * 8 + 4: return launch_gemv_t<EPI, 6, 4, true>(p, tpt, s);
+        }
+    }
     switch (sp.gpw * 8 + sp.ksplit) {
         case 1 * 8 + 1: return launch_gemv_t<EPI, 1, 1>(p, tpt, s);
         case 2 * 8 + 1: return launch_gemv_t<EPI, 2, 1>(p, tpt, s);
@@ -988,6 +1095,10 @@ int launch_gemv_e(const Params& p, int tpt, hipStream_t s) {
 
 bool gemv_supported(int64_t K, int64_t group_size) {
     return mfma_supported(K, group_size) && gemv_split((int)(K / group_size)).gpw > 0;
+}
+
+bool gemv_whole_split(int64_t K, int64_t group_size) {
+    return gemv_supported(K, group_size) && !gemv_split((int)(K / group_size)).ragged;
 }
 
 bool mfma_supported(int64_t K, int64_t group_size, bool e2m1) {
@@ -1042,7 +1153,7 @@ int launch_grouped_gemv_tpt(const GroupedArgs& a, int tpt, hipStream_t s) {
         return W4A8_ERR_INVALID;
     }
     if (!gemv_supported(a.K, a.group_size)) {
-        set_error("gemv grouped GEMM: K / group_size must be one of 1,2,3,4,6,8,12,16,32");
+        set_error("gemv grouped GEMM: K / group_size must be 1..24 or 32");
         return W4A8_ERR_INVALID;
     }
     if (a.e2m1) {

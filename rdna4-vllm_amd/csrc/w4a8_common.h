@@ -105,21 +105,21 @@ __device__ __forceinline__ float e4m3_pair_sum(float t, uint32_t a, uint32_t b) 
     return t;
 }
 
-// 16-entry byte lookup of each byte of x (values 0..15) in table t.
-// v_perm_b32 selects from 8 bytes; entries 8..15 come from a second select, and the
-// third select turns (x + 5) >= 13 into an all-ones byte mask for x >= 8.
+// 16-entry byte lookup of the low nibble of each byte of x in table t.
+// v_perm_b32 selects from 8 bytes: entries 0..7 and 8..15 by the low three bits, then byte i
+// of one or the other by bit 3 (six operations a dword: and, perm, perm, shift, and-or, perm).
 __device__ __forceinline__ uint32_t lut16(uint32_t x, uint4 t) {
-    const uint32_t a = __builtin_amdgcn_perm(t.y, t.x, x);
-    const uint32_t b = __builtin_amdgcn_perm(t.w, t.z, x ^ 0x08080808u);
-    const uint32_t m = __builtin_amdgcn_perm(0u, 0u, x + 0x05050505u);
-    return (a & ~m) | (b & m);
+    const uint32_t j = x & 0x07070707u;
+    const uint32_t a = __builtin_amdgcn_perm(t.y, t.x, j);
+    const uint32_t b = __builtin_amdgcn_perm(t.w, t.z, j);
+    return __builtin_amdgcn_perm(b, a, ((x >> 1) & 0x04040404u) | 0x03020100u);
 }
 
 // One int32 of 8 nibbles (k = 0..7) -> 8 e4m3 bytes in k8-interleave order:
 // lo = {k0,k2,k4,k6}, hi = {k1,k3,k5,k7}.
 __device__ __forceinline__ void decode8(uint32_t w, uint4 t, uint32_t& lo, uint32_t& hi) {
-    lo = lut16(w & 0x0F0F0F0Fu, t);
-    hi = lut16((w >> 4) & 0x0F0F0F0Fu, t);
+    lo = lut16(w, t);        // (reads the low four bits of a byte only)
+    hi = lut16(w >> 4, t);
 }
 
 __device__ __forceinline__ uint4 load_table(int idx) {

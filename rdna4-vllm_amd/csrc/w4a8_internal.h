@@ -223,8 +223,11 @@ bool prefill_supported(int64_t K, int64_t group_size, bool e2m1);   // g128, K <
 int launch_grouped_gemv_tpt(const GroupedArgs& a, int tiles_per_team, hipStream_t stream);
 // the matrix-core tiles take the shape (int4: group 128; E2M1: groups of 32, 64 or 128)
 bool mfma_supported(int64_t K, int64_t group_size, bool e2m1 = false);
-// mfma_supported and K / group_size in {1,2,3,4,6,8,12,16,32} (split-K table of the GEMV)
+// mfma_supported and K / group_size in 1..24 or 32
 bool gemv_supported(int64_t K, int64_t group_size);
+// ... in {1,2,3,4,6,8,12,16,32}, which the GEMV's waves split evenly: it then also quantises rows
+// itself and reads fragment-layout weights
+bool gemv_whole_split(int64_t K, int64_t group_size);
 
 // Whole-layer decode GEMV on fragment-layout weights (decode_gemv.hip): each work-group
 // groups the slots by expert from topk_ids itself and quantises its activation rows in
