@@ -193,6 +193,7 @@ bool dense_split_leads(int64_t M, int64_t N, int64_t K) {
 }
 
 int launch_dense_split(const GroupedArgs& a, hipStream_t s) {
+    if (a.P == 0) return W4A8_OK;
     SplitParams p;
     p.xq = a.x_fp8;
     p.asc = a.act_scales;

@@ -65,3 +65,11 @@ def test_bf16_rows_equal_their_fp16_cast(M, N, K):
     a = torch.ops.vllm.w4a8_dense_apply(x, *args)
     b = torch.ops.vllm.w4a8_dense_apply(x.to(torch.float16), *args)
     assert torch.equal(a, b)
+
+
+# no rows: an empty result and no launch, whichever kernel the sizes choose
+@pytest.mark.parametrize("N,K", [(256, 1024), (256, 1152), (520, 12288), (12296, 4352)])
+@pytest.mark.parametrize("kernel", ["prefill_wmma_ashuffle", "decode_gemv"])
+def test_no_rows(N, K, kernel):
+    x, w, s, z = _case(0, N, K, True, N + K)
+    assert tuple(W.mmq_fp8_gemm(x, w, s, kernel=kernel, w_zeros=z).shape) == (0, N)
