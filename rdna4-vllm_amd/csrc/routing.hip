@@ -354,10 +354,10 @@ __global__ void __launch_bounds__(kAlignThreads) align_quant_kernel(
     const int32_t* __restrict__ emap, int emap_len, int32_t* __restrict__ sorted_ids,
     int64_t sorted_len, int32_t* __restrict__ expert_ids, int32_t* __restrict__ ntp,
     int32_t* __restrict__ slot_to_row, const void* __restrict__ x, int64_t rows, int K,
-    uint8_t* __restrict__ xq, float* __restrict__ xs, float* __restrict__ gsum) {
+    uint8_t* __restrict__ xq, float* __restrict__ xs, bool k8, float* __restrict__ gsum) {
     if (blockIdx.x > 0) {
         const int64_t row = (int64_t)(blockIdx.x - 1) * (kAlignThreads / 64) + (threadIdx.x >> 6);
-        if (row < rows) quantize_row<BF16>(x, row, K, xq, xs, true, gsum, threadIdx.x & 63);
+        if (row < rows) quantize_row<BF16>(x, row, K, xq, xs, k8, gsum, threadIdx.x & 63);
         return;
     }
     align_small_body(ids, numel, E, block_m, emap, emap_len, sorted_ids, sorted_len, expert_ids,
@@ -451,7 +451,7 @@ int launch_align_quant(const int32_t* ids, int64_t numel, int64_t E, int64_t blo
                        int64_t sorted_len,
                        int32_t* expert_ids, int32_t* ntp, int32_t* slot_to_row,
                        const void* x, bool x_bf16, int64_t rows, int64_t K, uint8_t* xq,
-                       float* xs, float* gsum, hipStream_t stream) {
+                       float* xs, bool k8, float* gsum, hipStream_t stream) {
     if (E > kMaxExperts || numel > kChunk) {
         set_error("align_quant: needs num_experts <= 1024 and numel <= 1024");
         return W4A8_ERR_INVALID;
@@ -460,11 +460,11 @@ int launch_align_quant(const int32_t* ids, int64_t numel, int64_t E, int64_t blo
     if (x_bf16)
         align_quant_kernel<true><<<grid, kAlignThreads, 0, stream>>>(
             ids, numel, (int)E, block_m, emap, (int)emap_len, sorted_ids, sorted_len, expert_ids,
-            ntp, slot_to_row, x, rows, (int)K, xq, xs, gsum);
+            ntp, slot_to_row, x, rows, (int)K, xq, xs, k8, gsum);
     else
         align_quant_kernel<false><<<grid, kAlignThreads, 0, stream>>>(
             ids, numel, (int)E, block_m, emap, (int)emap_len, sorted_ids, sorted_len, expert_ids,
-            ntp, slot_to_row, x, rows, (int)K, xq, xs, gsum);
+            ntp, slot_to_row, x, rows, (int)K, xq, xs, k8, gsum);
     return check_launch("align_quant_kernel");
 }
 

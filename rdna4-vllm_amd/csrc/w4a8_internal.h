@@ -96,7 +96,7 @@ int launch_topk_softmax(const float* logits, int64_t T, int64_t E, int64_t top_k
                         uint8_t* xq = nullptr, float* xs = nullptr, float* gsum = nullptr);
 size_t align_workspace_bytes(int64_t numel, int64_t num_experts);
 // Decode prologue in one launch (numel <= 1024): the single-work-group align plus per-row
-// act-quant of x (k8-interleaved) with optional group sums.
+// act-quant of x (k8: k8-interleaved, else natural order) with optional group sums.
 // emap (emap_len entries) maps routed ids to local experts in [0, E); slots without a
 // local expert are dropped.
 int launch_align_quant(const int32_t* ids, int64_t numel, int64_t E, int64_t block_m,
@@ -104,7 +104,7 @@ int launch_align_quant(const int32_t* ids, int64_t numel, int64_t E, int64_t blo
                        int64_t sorted_len,
                        int32_t* expert_ids, int32_t* ntp, int32_t* slot_to_row,
                        const void* x, bool x_bf16, int64_t rows, int64_t K, uint8_t* xq,
-                       float* xs, float* gsum, hipStream_t stream);
+                       float* xs, bool k8, float* gsum, hipStream_t stream);
 int launch_align(const int32_t* topk_ids, int64_t numel, int64_t E, int64_t block_m,
                  const int32_t* expert_map, int64_t emap_len, int32_t* sorted_ids,
                  int64_t sorted_len,

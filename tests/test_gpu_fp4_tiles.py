@@ -66,7 +66,9 @@ def test_tiles_match_scalar(N, K, block_m, kind):
 
 
 @pytest.mark.parametrize("H,I,T", [(2880, 2880, 1), (2880, 2880, 33), (2880, 2880, 170), (128, 160, 5),
-                                   (1024, 544, 70)])
+                                   (1024, 544, 70),
+                                   # the last and first sizes of the shared align and row launch
+                                   (160, 128, 256), (160, 128, 257), (4096, 128, 9), (4128, 128, 9)])
 @pytest.mark.parametrize("act,bias,dtype", [("swigluoai", True, torch.bfloat16),
                                             ("silu", True, torch.float16),
                                             ("swigluoai", False, torch.float32)])
