@@ -979,8 +979,8 @@ int launch_mfma_e(const Params& p, hipStream_t s) {
     return launch_mfma_b<EPI>(p, s);
 }
 
-// Split of the K groups over waves: G == GPW * KSPLIT for the shapes below; others up to 32
-// take the next larger split with the last wave's missing groups masked (ragged), and past that
+// Split of the K groups over waves: G == GPW * KSPLIT for the shapes below; others up to 24
+// take the next larger split with the last waves' missing groups masked (ragged), and past that
 // the matrix-core tiles. E = 128, top-8, hidden 2304 (18 groups), intermediate 896 (7), T = 24,
 // the layer: 140 us on the tiles (87.6 + 43.4), 95 here; T = 1 44 / 41, T = 96 185 / 120.
 struct GemvSplit {

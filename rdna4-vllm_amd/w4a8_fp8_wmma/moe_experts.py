@@ -36,7 +36,7 @@ logger = logging.getLogger(__name__)
 AWQ_NIBBLE_OF = (0, 4, 1, 5, 2, 6, 3, 7)
 MOE_KERNEL_NAMES = ("scalar", "wmma", "gemv")        # moe_experts.py:72
 # gated activations between the GEMMs: SiLU (fused into gemm1 on the whole-layer path) and
-# gpt-oss's swigluoai (op by op, as the reference's mxfp4 hook runs it)
+# gpt-oss's swigluoai
 GATED_ACTIVATIONS = ("silu", "swigluoai")
 GEMV_MAX_M = 96                                      # moe_experts.py:563
 APPLY_CHUNK = 4096                                   # moe_experts.py:533
