@@ -871,6 +871,15 @@ __global__ void __launch_bounds__(256, 2) grouped_gemv_kernel(Params p, int tpt)
                     for (int r = 0; r < 4; ++r) run[f][r] = fmaf(acc[r], s, run[f][r]);
                 }
             }
+            // Three groups a wave: the folds stay before the branches below. Moved into them by the
+            // compiler (not with the other splits, where the pin costs 2%), an MFMA's result had no
+            // reader on the path that stores no tile, and no wait stood between it and the next
+            // write of its registers there, an address of issue(). No call takes that path; the
+            // code relies on none.
+            if constexpr (RAG && GPW == 3) {
+#pragma unroll
+                for (int f = 0; f < C::FR; ++f) pin_v4f(run[f]);
+            }
             if (c % C::NB != C::NB - 1) return;
             // tile set complete
 #pragma unroll

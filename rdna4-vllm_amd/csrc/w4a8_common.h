@@ -57,6 +57,16 @@ constexpr int kCpolSc1 = 16;
 using v4f = float __attribute__((ext_vector_type(4)));
 using v16f = float __attribute__((ext_vector_type(16)));
 
+// v is computed here: the compiler may not move what makes it past this point.
+__device__ __forceinline__ void pin_v4f(v4f& v) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        float t = v[r];
+        asm volatile("" : "+v"(t));
+        v[r] = t;
+    }
+}
+
 // Nibble -> e4m3 byte tables, 4 dwords each (entry i in byte i%4 of dword i/4).
 // Table z < 16 holds e4m3(n - z) for n = 0..15; table 16 holds e4m3 of the OCP E2M1
 // codebook {0,.5,1,1.5,2,3,4,6,-0,-.5,...,-6}. Every entry is exact in e4m3.
