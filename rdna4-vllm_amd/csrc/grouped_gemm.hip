@@ -1047,7 +1047,14 @@ int launch_gemv_t(const Params& p, int tpt, hipStream_t s) {
     using C = GemvCfg<EPI, GPW, KSPLIT, RAG>;
     const int ncols = C::kSilu ? p.N / 2 : p.N;
     const int ntiles = (ncols + 15) / 16;
-    if (tpt <= 0) tpt = gemv_default_tpt(p, ntiles, GPW * C::NF * 1024, C::TEAMS, RAG ? 384 : 512);
+    if (tpt <= 0) {
+        tpt = gemv_default_tpt(p, ntiles, GPW * C::NF * 1024, C::TEAMS, RAG ? 384 : 512);
+        // With eight gate and up tiles, the partial sums (64 KB) beside the table leave a CU one
+        // work-group; four tiles lead there with three and four groups a wave: E = 64, top-8,
+        // intermediate 768, T = 16, the layer with 13 groups 64.9 -> 51.7 us (63.5 on the tiles),
+        // with 9 44.9 -> 41.7 (48.0); with 18, five a wave, 81 -> 86.
+        if (RAG && C::kSilu && GPW <= 4) tpt = std::min(tpt, 4);
+    }
     tpt = std::min(tpt, kGemvMaxTiles);
     const size_t lds = KSPLIT > 1 ? (size_t)4 * tpt * C::NF * 64 * sizeof(v4f) : 0;
     const dim3 grid((unsigned)((ntiles + C::TEAMS * tpt - 1) / (C::TEAMS * tpt)),

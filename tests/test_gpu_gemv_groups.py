@@ -3,10 +3,14 @@ float64 product of the same quantised operands.
 
 Products are exact and summed in fp32, then one rounding to fp16: half an fp16 ulp (2^-11) plus
 the sums' rounding, below 2^-11 of the largest output at these sizes: 2^-10 of the largest."""
+import numpy as np
 import pytest
 import torch
 
+import bench
+import oracle as O
 import w4a8_fp8_wmma as W
+from w4a8_fp8_wmma import moe_experts
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -45,3 +49,46 @@ def test_uneven_groups(G, asym, T, N, block_m):
         assert float((got[p] - ref).abs().max() / ref.abs().max()) <= 2.0 ** -10
         rows += 1
     assert rows == T * k
+
+
+# each split in gemm1 (gate and up, SiLU) and in gemm2 (slot outputs); one to four tiles a
+# work-group in gemm1, up to eight in gemm2
+@pytest.mark.parametrize("H,I", [(640, 128), (896, 640), (1152, 896), (1280, 1152), (1408, 1280), (1664, 1408),
+                                 (1920, 1792), (2176, 2176), (2304, 2560), (2688, 2688), (3072, 3072)])
+@pytest.mark.parametrize("asym", [True, False])
+@pytest.mark.parametrize("T,E", [(3, 4), (40, 64)])
+def test_decode_layer_equals_composition(H, I, asym, T, E):
+    """A decode layer on the op layout against gemm (checked above), silu_and_mul, gemm and
+    gather-reduce. The composition rounds y to fp16 (half an ulp: 2^-11 of each term) and both
+    round the output (2^-11 each): within 2^-9 of the largest output; a wrong gate, up, scale or
+    zero-point is off by its own size."""
+    g = torch.Generator(device=DEV).manual_seed(H + I + T + asym)
+    words = lambda *s: torch.randint(-2**31, 2**31 - 1, s, generator=g, device=DEV,
+                                     dtype=torch.int64).to(torch.int32)
+    scales = lambda *s: (torch.rand(s, generator=g, device=DEV) * 0.015 + 0.005).to(torch.float16)
+    w13, w2 = words(E, 2 * I, H // 8), words(E, H, I // 8)
+    s13, s2 = scales(E, 2 * I, H // 128), scales(E, H, I // 128)
+    z13, z2 = (words(E, 2 * I // 8, H // 128), words(E, H // 8, I // 128)) if asym else (None, None)
+    x = (torch.randn((T, H), generator=g, device=DEV) * 0.1).to(torch.float16)
+    ids = torch.rand((T, E), generator=g, device=DEV).argsort(1)[:, :2].to(torch.int32).contiguous()
+    tw = torch.rand((T, 2), generator=g, device=DEV)
+    out = W.moe_apply(x, w13, w2, s13, s2, z13, z2, tw, ids).float()
+    ref = moe_experts._run_unfused(x, w13, w2, s13, s2, z13, z2, tw.reshape(-1), ids, 2, E, None,
+                                   "gemv", False, None, None, 16).float()
+    assert torch.isfinite(out).all() and float((out - ref).abs().max()) <= 2.0 ** -9 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("H,I", [(2304, 896), (640, 1152), (1664, 2816)])
+@pytest.mark.parametrize("asym", [True, False])
+@pytest.mark.parametrize("T", [3, 24])
+def test_decode_layer_vs_oracle(H, I, asym, T):
+    """A decode layer with uneven K groups in both GEMMs: SiLU and slot outputs, the layer's bar."""
+    ws = bench.make_weights(dict(T=T, H=H, E=8, k=2, I=I, g=128, routing="uniform"), H + T, DEV)
+    z13, z2 = (ws["z13"], ws["z2"]) if asym else (None, None)
+    x, logits = bench.make_inputs(dict(T=T, H=H, E=8, k=2, I=I, g=128, routing="uniform"), I + T, DEV)
+    tw, ids = W.fused_topk(None, logits, 2, True)
+    out = W.moe_apply(x, ws["w13"], ws["w2"], ws["s13"], ws["s2"], z13, z2, tw, ids)
+    n = lambda t: None if t is None else t.cpu().numpy()
+    ref = O.moe_layer(n(x.float()), n(ws["w13"]), n(ws["s13"]), n(z13), n(ws["w2"]), n(ws["s2"]),
+                      n(z2), n(tw), n(ids), 128, round_y_fp16=False)
+    assert np.abs(n(out.float()) - ref).max() <= 1e-2 * np.abs(ref).max()
