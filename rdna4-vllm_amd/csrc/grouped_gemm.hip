@@ -1176,6 +1176,13 @@ int launch_grouped_gemv_tpt(const GroupedArgs& a, int tpt, hipStream_t s) {
         set_error("gemv grouped GEMM: E2M1 weights run on the matrix-core tiles");
         return W4A8_ERR_INVALID;
     }
+    // uneven K groups keep the bounds of the tiles that ran them (32-bit offsets here as there)
+    if (!gemv_whole_split(a.K, a.group_size) &&
+        (a.block_m % 16 != 0 || a.N * (a.K / 2) >= (int64_t)1 << 31 || a.x_rows * a.K >= (int64_t)1 << 31)) {
+        set_error("gemv grouped GEMM: this number of K groups needs block_m a multiple of 16, expert "
+                  "slices and rows below 2 GiB");
+        return W4A8_ERR_INVALID;
+    }
     if (a.w_frag && (a.N % 16 != 0 || (a.epi == Epi::kSiluHalf && (a.N / 2) % 16 != 0))) {
         set_error("gemv grouped GEMM: fragment-layout weights need 16-row aligned halves");
         return W4A8_ERR_INVALID;

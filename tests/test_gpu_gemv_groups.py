@@ -92,3 +92,22 @@ def test_decode_layer_vs_oracle(H, I, asym, T):
     ref = O.moe_layer(n(x.float()), n(ws["w13"]), n(ws["s13"]), n(z13), n(ws["w2"]), n(ws["s2"]),
                       n(z2), n(tw), n(ids), 128, round_y_fp16=False)
     assert np.abs(n(out.float()) - ref).max() <= 1e-2 * np.abs(ref).max()
+
+
+def test_bounds_of_the_tiles_stay():
+    """Where the tiles refused a call of these sizes the GEMV refuses it too: weights of 2 GiB an
+    expert (its offsets are 32-bit), blocks of 8 rows."""
+    K = 5 * 128
+    x = torch.zeros((16, K), dtype=torch.float16, device=DEV)
+    route = [torch.zeros(n, dtype=torch.int32, device=DEV) for n in (16, 2, 1)]
+
+    def call(N, block_m):
+        w = torch.empty((1, N, K // 8), dtype=torch.int32, device=DEV)
+        s = torch.empty((1, N, 5), dtype=torch.float16, device=DEV)
+        return W.mmq_fp8_moe_gemm(x, w, s, route[0], route[1][:16 // block_m].contiguous(), route[2], 1, block_m,
+                                  kernel="gemv")
+
+    assert tuple(call(64, 16).shape) == (16, 64)
+    for N, block_m in ((64, 8), (2 ** 32 // K + 8, 16)):
+        with pytest.raises(RuntimeError, match="gemv grouped GEMM"):
+            call(N, block_m)
