@@ -52,12 +52,13 @@ __device__ __forceinline__ void quantize_row_regs(const RowRegs& rr, int64_t row
                                                   float* __restrict__ gsum, int lane);
 
 // A row of up to kBlockRowMaxK values by a work-group of four waves (row start 16-byte aligned):
-// wave w holds the 512-wide passes w, w + 4, ... in registers, the absmaxes meet in LDS.
+// wave w holds the 512-wide passes w, w + 4, ... in registers, the absmaxes meet in LDS. (No
+// group sums: the tiles that read them take rows of up to 4096 values.)
 constexpr int kBlockRowMaxK = 16384;
 template <bool BF16>
 __device__ __forceinline__ void quantize_row_block(const void* __restrict__ x, int64_t row, int K,
                                                    uint8_t* __restrict__ q, float* __restrict__ scales,
-                                                   bool k8, float* __restrict__ gsum, float* s_amax);
+                                                   bool k8, float* s_amax);
 
 // Group sum of one 512-wide pass (lanes 16j..16j+15 hold group k/128): fixed-order tree.
 __device__ __forceinline__ void row_group_sum(uint32_t lo, uint32_t hi, int64_t row, int K, int k,
@@ -187,7 +188,7 @@ __device__ __forceinline__ float absmax_u4(const uint4& v) {
 template <bool BF16>
 __device__ __forceinline__ void quantize_row_block(const void* __restrict__ x, int64_t row, int K,
                                                    uint8_t* __restrict__ q, float* __restrict__ scales,
-                                                   bool k8, float* __restrict__ gsum, float* s_amax) {
+                                                   bool k8, float* s_amax) {
     constexpr int kMaxPass = kBlockRowMaxK / 2048;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int npass = (K + 511) / 512;
@@ -228,7 +229,6 @@ __device__ __forceinline__ void quantize_row_block(const void* __restrict__ x, i
             }
             *reinterpret_cast<uint2*>(q + row * K + k) = make_uint2(lo, hi);
         }
-        if (gsum != nullptr) row_group_sum(lo, hi, row, K, k, gsum, lane);
     }
 }
 

@@ -102,7 +102,7 @@ int run_grouped(GroupedArgs& a, int64_t kernel, void* ws, size_t ws_bytes, hipSt
     const bool prefill = tiles && prefill_supported(a.K, a.group_size, a.e2m1);
     const bool wide = tiles && dense;
     const bool split = wide && dense_split_leads(a.P, a.N, a.K);
-    a.act_group_sums = (prefill || wide) && !split ? gsum : nullptr;
+    a.act_group_sums = prefill && !wide ? gsum : nullptr;
     if (int rc = launch_act_quant(a.x, a.x_bf16, a.x_rows, a.K, a.x_fp8, a.act_scales, k8, s,
                                   filter ? a.sorted_ids : nullptr, filter ? a.ntp : nullptr,
                                   a.num_valid, a.act_group_sums))

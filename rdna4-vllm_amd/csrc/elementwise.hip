@@ -28,12 +28,11 @@ __global__ void __launch_bounds__(256) act_quant_kernel(
 template <bool BF16>
 __global__ void __launch_bounds__(256) act_quant_block_kernel(
     const void* __restrict__ x, int K, uint8_t* __restrict__ q, float* __restrict__ scales, bool k8,
-    const int32_t* __restrict__ sorted_ids, const int32_t* __restrict__ ntp, int64_t num_valid,
-    float* __restrict__ gsum) {
+    const int32_t* __restrict__ sorted_ids, const int32_t* __restrict__ ntp, int64_t num_valid) {
     __shared__ float s_amax[4];
     const int64_t row = blockIdx.x;
     if (sorted_ids != nullptr && (row >= ntp[0] || sorted_ids[row] >= num_valid)) return;
-    quantize_row_block<BF16>(x, row, K, q, scales, k8, gsum, s_amax);
+    quantize_row_block<BF16>(x, row, K, q, scales, k8, s_amax);
 }
 
 // One thread per (row, 8-wide k chunk): decode 8 nibbles through the same table path the
@@ -281,13 +280,13 @@ int launch_act_quant(const void* x, bool x_bf16, int64_t rows, int64_t K, uint8_
     }
     dim3 grid(blocks_for(rows, kWavesPerBlock)), block(64 * kWavesPerBlock);
     if (K > RowRegs::kMaxPass * 512 && K <= kBlockRowMaxK && K % 8 == 0 && rows < ((int64_t)1 << 31) &&
-        reinterpret_cast<uintptr_t>(x) % 16 == 0) {
+        group_sums == nullptr && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
         if (x_bf16)
             act_quant_block_kernel<true><<<(unsigned)rows, 256, 0, stream>>>(
-                x, (int)K, x_fp8, scales, k8, sorted_ids, ntp, num_valid, group_sums);
+                x, (int)K, x_fp8, scales, k8, sorted_ids, ntp, num_valid);
         else
             act_quant_block_kernel<false><<<(unsigned)rows, 256, 0, stream>>>(
-                x, (int)K, x_fp8, scales, k8, sorted_ids, ntp, num_valid, group_sums);
+                x, (int)K, x_fp8, scales, k8, sorted_ids, ntp, num_valid);
         return check_launch("act_quant_block_kernel");
     }
     if (x_bf16)

@@ -97,22 +97,6 @@ __global__ void __launch_bounds__(256) grouped_scalar_kernel(Params p) {
 }
 
 // =====================================================================================
-// MFMA helpers
-// =====================================================================================
-// 4 words (32 nibbles, k = 0..31 of a fragment) -> 8 dwords of e4m3 (k8-interleaved).
-__device__ __forceinline__ v8i decode_frag(uint4 wv, uint4 t) {
-    uint32_t o[8];
-    decode8(wv.x, t, o[0], o[1]);
-    decode8(wv.y, t, o[2], o[3]);
-    decode8(wv.z, t, o[4], o[5]);
-    decode8(wv.w, t, o[6], o[7]);
-    v8i r;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) r[i] = (int)o[i];
-    return r;
-}
-
-// =====================================================================================
 // MFMA tiled (prefill) kernel
 // =====================================================================================
 constexpr int kLdsStride = kGroup + 16;

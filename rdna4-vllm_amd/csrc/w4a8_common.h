@@ -137,6 +137,38 @@ __device__ __forceinline__ uint4 load_table(int idx) {
                       g_decode_tables[idx][2], g_decode_tables[idx][3]);
 }
 
+// 4 words (32 nibbles, k = 0..31 of a fragment) -> 8 dwords of e4m3 (k8-interleaved).
+__device__ __forceinline__ v8i decode_frag(uint4 wv, uint4 t) {
+    uint32_t o[8];
+    decode8(wv.x, t, o[0], o[1]);
+    decode8(wv.y, t, o[2], o[3]);
+    decode8(wv.z, t, o[4], o[5]);
+    decode8(wv.w, t, o[6], o[7]);
+    v8i r;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r[i] = (int)o[i];
+    return r;
+}
+
+// decode_frag with lut16's masks in registers: gfx950's three-operand instructions take no
+// literals, so the compiler can fuse the and with the or only where the masks are no constants to
+// it (13 instead of 15 operations a word).
+struct DecodeMasks {
+    uint32_t c7, c4, c3;
+};
+__device__ __forceinline__ DecodeMasks decode_masks() {
+    return {opaque_u32(0x07070707u), opaque_u32(0x04040404u), opaque_u32(0x03020100u)};
+}
+__device__ __forceinline__ v8i decode_frag(const u32x4& w, const uint4& t, const DecodeMasks& m) {
+    auto lut = [&](uint32_t x) __attribute__((always_inline)) {
+        const uint32_t j = x & m.c7;
+        const uint32_t a = __builtin_amdgcn_perm(t.y, t.x, j);
+        const uint32_t b = __builtin_amdgcn_perm(t.w, t.z, j);
+        return (int)__builtin_amdgcn_perm(b, a, ((x >> 1) & m.c4) | m.c3);
+    };
+    return v8i{lut(w.x), lut(w.x >> 4), lut(w.y), lut(w.y >> 4), lut(w.z), lut(w.z >> 4), lut(w.w), lut(w.w >> 4)};
+}
+
 // Decode-table index for output row n, group g of one expert's packed zero-points
 // (E, N/8, G) (moe_kernel.hip:172-176: (z[n/8][g] >> 4*(n%8)) & 0xF).
 __device__ __forceinline__ int table_index(const int* __restrict__ zeros_e, int n, int g,
