@@ -6,10 +6,10 @@
 // A work-group owns 16 MT rows x 16 columns; its eight waves take an eighth of the K groups
 // each, so a dense GEMM whose output has few tiles still keeps every CU streaming weights, and
 // no wave waits for another until the partial sums meet in LDS at the end (added in wave order).
-// Rows come quantised (act_quant_kernel). Per group, as in the GEMVs: one 16x16x128 MFMA a block
-// on the raw nibbles, the zero-point term from the rows' sums (an MFMA against ones), the fp16
-// scale fold. Two column fragments a work-group measured slower at every size (half the
-// work-groups; registers): (4096, 12288) M = 64 53 -> 121 us.
+// Rows come quantised (act_quant_kernel). Per group the weights are decoded to e4m3(n - z) (raw
+// nibbles lose precision, see wide_tiles.hip), then one 16x16x128 MFMA a block and the fp16 scale
+// fold. Two column fragments a work-group measured slower at every size (half the
+// work-groups; registers): (4096, 12288) M = 64 53 -> 121 us on raw nibbles.
 #include <algorithm>
 #include <type_traits>
 
@@ -20,7 +20,6 @@ namespace {
 
 constexpr int kDsWaves = 8;
 constexpr int NT = 1;                       // column fragments of a work-group
-constexpr uint32_t kDsOnes = 0x38383838u;   // four e4m3 bytes of 1.0
 
 struct SplitParams {
     const uint8_t* xq;     // (M, K) e4m3, k8-interleaved
@@ -32,9 +31,11 @@ struct SplitParams {
     int M, N, K, G;
 };
 
-template <int MT>
+// ZP: weights with zero-points (else the zero point is 8)
+template <int MT, bool ZP>
 __global__ void __launch_bounds__(64 * kDsWaves, 2) dense_split_kernel(SplitParams p) {
     __shared__ v4f s_part[kDsWaves][MT * NT][64];
+    __shared__ uint4 s_lut[ZP ? 16 : 1];        // e4m3(n - z) tables
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int q = lane >> 4, c16 = lane & 15;
@@ -64,7 +65,7 @@ __global__ void __launch_bounds__(64 * kDsWaves, 2) dense_split_kernel(SplitPara
     constexpr int D = 4;                 // weight groups in flight
     constexpr int DA = MT > 2 ? 2 : 4;   // row groups in flight (their registers grow with MT)
     u32x4 bw[D][NT], ar[DA][MT][2];
-    uint32_t sv[D][NT], zv[D][NT];
+    uint32_t sv[D][NT], zv[ZP ? D : 1][NT];
     auto issue_b = [&](int g, auto sc) __attribute__((always_inline)) {
         constexpr int s = decltype(sc)::value;
         const uint32_t gg = (uint32_t)min(g, G - 1);         // past the end: never used
@@ -72,7 +73,7 @@ __global__ void __launch_bounds__(64 * kDsWaves, 2) dense_split_kernel(SplitPara
         for (int j = 0; j < NT; ++j) {
             bw[s][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wb + opaque_u32(woff[j] + gg * 64u)));
             sv[s][j] = *reinterpret_cast<const uint16_t*>(sb + opaque_u32(soff[j] + gg * 2u));
-            zv[s][j] = p.z ? *reinterpret_cast<const uint32_t*>(zb + opaque_u32(zoff[j] + gg * 4u)) : 0u;
+            if constexpr (ZP) zv[s][j] = *reinterpret_cast<const uint32_t*>(zb + opaque_u32(zoff[j] + gg * 4u));
         }
     };
     auto issue_a = [&](int g, auto sc) __attribute__((always_inline)) {
@@ -90,34 +91,28 @@ __global__ void __launch_bounds__(64 * kDsWaves, 2) dense_split_kernel(SplitPara
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) run[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    const int one = (int)kDsOnes;
-    const v8i ones = {one, one, one, one, one, one, one, one};
+    const DecodeMasks masks = decode_masks();
+    const uint4 t8 = load_table(8);
+    if (ZP && threadIdx.x < 16) s_lut[threadIdx.x] = load_table(threadIdx.x);
     auto step = [&](int g, auto sc) __attribute__((always_inline)) {
         constexpr int s = decltype(sc)::value, sa_ = s % DA;
         v8i bf[NT];
-        float sf[NT], zf[NT];
+        float sf[NT];
 #pragma unroll
         for (int j = 0; j < NT; ++j) {
-            bf[j] = spread_nibbles(make_uint4(bw[s][j].x, bw[s][j].y, bw[s][j].z, bw[s][j].w));
+            const uint4 t = ZP ? s_lut[(zv[ZP ? s : 0][j] >> zsh[j]) & 0xFu] : t8;
+            bf[j] = decode_frag(bw[s][j], t, masks);
             sf[j] = __half2float(__ushort_as_half((unsigned short)sv[s][j]));
-            zf[j] = p.z ? (float)((zv[s][j] >> zsh[j]) & 0xFu) : 8.0f;
         }
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
             const u32x4 lo = ar[sa_][i][0], hi = ar[sa_][i][1];
             const v8i af = {(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w, (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-            // 2^-9 x the group sums of rows 4 q .. 4 q + 3 (zero-point term)
-            v4f sa = mfma_16x16x128(af, ones, v4f{0.f, 0.f, 0.f, 0.f});
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sa[r] *= 1.0f / kNibbleScale;
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
-                v4f acc = mfma_16x16x128(af, bf[j], v4f{0.f, 0.f, 0.f, 0.f});
+                const v4f acc = mfma_16x16x128(af, bf[j], v4f{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    acc[r] = fmaf(-zf[j], sa[r], acc[r]);
-                    run[i][j][r] = fmaf(acc[r], sf[j], run[i][j][r]);
-                }
+                for (int r = 0; r < 4; ++r) run[i][j][r] = fmaf(acc[r], sf[j], run[i][j][r]);
             }
         }
         issue_a(g + DA, sc);
@@ -138,6 +133,7 @@ __global__ void __launch_bounds__(64 * kDsWaves, 2) dense_split_kernel(SplitPara
     fill(S1{});
     fill(S2{});
     fill(S3{});
+    if constexpr (ZP) lds_barrier();   // the tables are written
     const int nq = (ge - gb) / D, rem = (ge - gb) % D;
     int g = gb;
     for (int it = 0; it < nq; ++it, g += D) {
@@ -169,7 +165,7 @@ __global__ void __launch_bounds__(64 * kDsWaves, 2) dense_split_kernel(SplitPara
         for (int r = 0; r < 4; ++r) {
             const int m = row0 + 16 * (b / NT) + 4 * q + r;
             if (m < p.M && n < p.N)
-                p.out[(int64_t)m * p.N + n] = __float2half(as_f32(sum[r] * (p.asc[m] * kNibbleScale)));
+                p.out[(int64_t)m * p.N + n] = __float2half(as_f32(sum[r] * p.asc[m]));
         }
     }
 }
@@ -177,7 +173,8 @@ __global__ void __launch_bounds__(64 * kDsWaves, 2) dense_split_kernel(SplitPara
 template <int MT>
 int launch_split_t(const SplitParams& p, hipStream_t s) {
     const dim3 grid((unsigned)((p.N + 16 * NT - 1) / (16 * NT)), (unsigned)((p.M + 16 * MT - 1) / (16 * MT)));
-    dense_split_kernel<MT><<<grid, dim3(64 * kDsWaves), 0, s>>>(p);
+    if (p.z) dense_split_kernel<MT, true><<<grid, dim3(64 * kDsWaves), 0, s>>>(p);
+    else dense_split_kernel<MT, false><<<grid, dim3(64 * kDsWaves), 0, s>>>(p);
     return check_launch("dense_split_kernel");
 }
 
@@ -185,8 +182,8 @@ int launch_split_t(const SplitParams& p, hipStream_t s) {
 
 // While its 64-row x 16-column work-groups fit the CUs in one round and either the rows are few
 // or K is long: the wide tiles then have too few work-groups, each walking all of K (us, this /
-// 32 x 128 tiles: (N, K) = (4096, 12288) M = 17 32 / 64, M = 64 53 / 66, M = 96 (512 work-groups)
-// 83 / 67; (3008, 7040) M = 17 17 / 36; (1024, 4096) M = 17 15 / 23, M = 64 22 / 23).
+// 32 x 64 tiles: (N, K) = (4096, 12288) M = 17 23 / 52, M = 64 40 / 53; (2048, 6144) M = 17
+// 14 / 27, M = 128 25 / 29).
 bool dense_split_leads(int64_t M, int64_t N, int64_t K) {
     const int64_t wgs = (N + 15) / 16 * ((M + 63) / 64);
     return wgs <= device_cu_count() && (M <= 48 || K > 32 * kGroup);

@@ -92,6 +92,17 @@ def test_every_tile_past_its_tables(M, N, K, asym, rows):
     assert share <= LIMIT[rows] and worst <= 2.0 ** -10
 
 
+# the split-K kernel: 16 to 64 rows a work-group, fewer and more K groups than its waves' loads in
+# flight, uneven slices, K of few groups (some waves without any)
+@pytest.mark.parametrize("M,N,K", [(9, 520, 5120), (17, 4088, 4224), (40, 1000, 12288), (48, 4096, 1152),
+                                   (64, 1032, 8320), (100, 2040, 6144)])
+@pytest.mark.parametrize("asym", [True, False])
+@pytest.mark.parametrize("rows", ["normal", "non-negative"])
+def test_split_k_rounding(M, N, K, asym, rows):
+    share, worst = _misrounded(M, N, K, asym, rows)
+    assert share <= LIMIT[rows] and worst <= 2.0 ** -10
+
+
 @pytest.mark.parametrize("rows", ["normal", "non-negative"])
 def test_down_projection_of_a_prompt(rows):
     """96 groups: six tables of the largest tile, rows quantised a work-group each."""
