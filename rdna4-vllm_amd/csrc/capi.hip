@@ -59,10 +59,7 @@ int run_grouped(GroupedArgs& a, int64_t kernel, void* ws, size_t ws_bytes, hipSt
     const bool mfma = mfma_supported(a.K, a.group_size, a.e2m1);
     // E2M1 codebook weights take the matrix-core tiles (the GEMV feeds raw nibbles)
     bool gemv = gemv_supported(a.K, a.group_size) && !a.e2m1;
-    // One expert on identity rows (the dense op) with fp16 out: the GEMV streams the weights once
-    // per 16 rows; past 16 row blocks of 1024 columns (or their product) the wide tiles lead (us,
-    // GEMV / 32 x 128 tiles: (N, K) = (4096, 4096) M = 64 19 / 23, M = 96 27 / 23; (8192, 4096)
-    // M = 32 20 / 23, M = 64 25 / 23; (12288, 4096) M = 17 28 / 22; (1024, 4096) M = 256 20 / 24)
+    // one expert on identity rows with fp16 out: the dense op
     const bool dense = a.E == 1 && a.expert_ids == nullptr && a.epi == Epi::kHalf && !a.w_frag &&
                        wide_tiles_supported(a.x_rows, a.K, a.N, a.group_size, a.e2m1);
     Workspace w(ws, ws_bytes);
@@ -71,8 +68,9 @@ int run_grouped(GroupedArgs& a, int64_t kernel, void* ws, size_t ws_bytes, hipSt
     float* gsum = w.take<float>((size_t)(a.x_rows * ((a.K + 127) / 128)));
     const bool have_ws = !(a.x_rows > 0 && ws == nullptr) && w.ok();
     const bool whole = gemv_whole_split(a.K, a.group_size);
-    if (dense && have_ws && (!whole || (a.P + 15) / 16 * a.N > 16 * 1024)) gemv = false;
-    if (!have_ws && !whole) gemv = false;   // uneven groups take quantised rows (refused below)
+    // K groups that the GEMV's waves do not split evenly: the dense op runs its tiles under either
+    // name; without a workspace for the quantised rows the call is refused below
+    if (!whole && (dense || !have_ws)) gemv = false;
     // identity-gathered inputs (gemm2 / scatter) have one row per padded row: skip padding.
     const bool filter = a.identity_gather && a.sorted_ids != nullptr;
     if (kernel == W4A8_MOE_KERNEL_GEMV && gemv) {
@@ -93,8 +91,7 @@ int run_grouped(GroupedArgs& a, int64_t kernel, void* ws, size_t ws_bytes, hipSt
         set_error("workspace smaller than w4a8_moe_gemm_workspace_size()");
         return W4A8_ERR_WORKSPACE;
     }
-    // gemv for K-group counts outside its split-K table (or, dense, past its rows) runs the
-    // matrix-core tiles
+    // gemv for K-group counts outside its split-K table runs the matrix-core tiles
     const bool tiles = (kernel == W4A8_MOE_KERNEL_WMMA || kernel == W4A8_MOE_KERNEL_GEMV) && mfma;
     // E2M1 tiles take fp4 operands against activations in natural k order; every other
     // kernel (the scalar one included) takes k8-interleaved activations

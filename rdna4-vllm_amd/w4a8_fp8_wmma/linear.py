@@ -5,11 +5,12 @@
 (vllm_adapter.py:265-354): 2-D activations of any float dtype are cast to fp16, the result
 is (M, N) fp16. The kernel for a batch of M rows is picked by name:
 
-  * ``"decode_gemv"`` for M <= ``VLLM_ROCM_W4A8_DECODE_MAX_M`` at group 128, and (with the
-    variable unset) up to 2048 rows while the MFMA tile grid would hold fewer than 128
-    tiles (a K outside the GEMV's split-K table runs the MFMA tiles instead);
+  * ``"decode_gemv"`` for M <= ``VLLM_ROCM_W4A8_DECODE_MAX_M`` at group 128; with the variable
+    unset, where ``dense_kernel_for`` names it and the tiles do not lead (``_tiles_lead``). (K
+    group counts that the GEMV's waves do not split evenly run the tiles under either name.)
   * ``"prefill_wmma_ashuffle"`` otherwise (``"prefill_wmma"`` for group sizes other than 32 and
-    128, the reference's rule). On gfx950 both names run the fp8-MFMA tiles.
+    128, the reference's rule). On gfx950 both names run the fp8-MFMA tiles: at group 128 the
+    wide tiles, or the split-K kernel for some tens of rows.
 
 There is no Triton W4A16 fallback on this build: the Triton-layout arguments (``tri_bq``,
 ``tri_s``, ``tri_zp``) and the measured crossover ``cached_min_m`` are accepted for the call
@@ -33,16 +34,18 @@ from ._ops import dense_linear
 
 logger = logging.getLogger(__name__)
 
-#: Rows up to which the decode GEMV runs when VLLM_ROCM_W4A8_DECODE_MAX_M is unset. Measured
-#: on MI355X (HIP-graph replay) against the MFMA tiles for (N, K) = (1024, 2048), (4096, 4096),
-#: (12288, 4096), (4096, 12288): the GEMV leads through M = 128 on every shape.
+#: Rows up to which ``dense_kernel_for`` names the decode GEMV when VLLM_ROCM_W4A8_DECODE_MAX_M
+#: is unset, and past them up to DENSE_GEMV_MAX_M while ceil(N / 256) x ceil(M / 64) is below
+#: DENSE_MIN_TILES: half as many as MI355X has CUs.
 DECODE_MAX_M_DEFAULT = 128
-#: Past that (env unset) the GEMV still runs while the MFMA tile grid, ceil(N / 256) x
-#: ceil(M / 64) work-groups, holds fewer than half as many tiles as MI355X has CUs: such a grid
-#: leaves most CUs idle, and the GEMV measured faster on every shape above (e.g. (4096, 4096)
-#: at M = 256: 37.7 against 61.2 us; (1024, 2048) at M = 512: 14.3 against 38.0 us).
 DENSE_GEMV_MAX_M = 2048
 DENSE_TILE_ROWS, DENSE_TILE_COLS, DENSE_MIN_TILES = 64, 256, 128
+#: Past this product of 16-row blocks and columns the tiles lead the GEMV, which streams the
+#: weights once per 16 rows. GEMV time over tile time (MI355X, M = 17 .. 1024, N = 256 .. 28672)
+#: past it: K = 256 0.97 .. 1.4, K = 512 1.1 .. 1.6, K = 1024 1.05 .. 2.1, K = 2048 0.89 .. 2.5,
+#: K = 4096 1.04 .. 3.4; up to it 0.6 .. 1.1, up to 1.3 for few points. K = 128 gives a tile no
+#: second group to work on while the first arrives: 0.79 .. 1.07.
+TILES_LEAD_ROWS_COLS = 16 * 1024
 #: Symmetric int4 (vLLM ``uint4b8``) stores w + 8; the kernels' implicit zero point.
 UINT4B8_BIAS = 8
 
@@ -63,8 +66,7 @@ def decode_max_m() -> int:
 
 def dense_kernel_for(M: int, N: int, K: int, group_size: int) -> str:
     """The dense kernel name for an (M, N, K) GEMM with this group size (the ladder of
-    vllm_adapter.py:296-324 without its Triton band). A K outside the GEMV's split-K table
-    runs the MFMA tiles under either name (the C ABI's own fallback)."""
+    vllm_adapter.py:296-324 without its Triton band)."""
     if group_size == 128 and K % group_size == 0:
         if M <= decode_max_m():
             return "decode_gemv"
@@ -73,6 +75,23 @@ def dense_kernel_for(M: int, N: int, K: int, group_size: int) -> str:
                 and tiles < DENSE_MIN_TILES):
             return "decode_gemv"
     return "prefill_wmma_ashuffle" if group_size in (32, 128) else "prefill_wmma"
+
+
+def _tiles_lead(M: int, N: int, K: int) -> bool:
+    """Whether the tiles are the faster kernel at group 128 where dense_kernel_for names the GEMV.
+    (Up to 16 rows at K = 1024 .. 4096 have a GEMV of their own, which leads.)"""
+    if M <= 16 and N % 16 == 0 and K % 1024 == 0 and K <= 4096:
+        return False
+    return K > 128 and -(-M // 16) * N > TILES_LEAD_ROWS_COLS
+
+
+def _op_kernel(M: int, N: int, K: int, group_size: int) -> str:
+    """The kernel name the op runs: a boundary set in the environment decides alone."""
+    name = dense_kernel_for(M, N, K, group_size)
+    if (name == "decode_gemv" and "VLLM_ROCM_W4A8_DECODE_MAX_M" not in os.environ
+            and _tiles_lead(M, N, K)):
+        return "prefill_wmma_ashuffle"
+    return name
 
 
 def _dense_args(x2d, w_q, w_s, w_zp, tri_bq, tri_s, tri_zp, N, K, group_size, zero_points,
@@ -90,7 +109,7 @@ def _dense_args(x2d, w_q, w_s, w_zp, tri_bq, tri_s, tri_zp, N, K, group_size, ze
     if not use_zp and int(weight_type_bias) != UINT4B8_BIAS:
         raise ValueError("weights without zero points must be uint4b8 (bias 8), "
                          f"got bias {weight_type_bias}")
-    return x2d, w_q, w_s, w_zp if use_zp else None, dense_kernel_for(x2d.shape[0], N, K, group_size)
+    return x2d, w_q, w_s, w_zp if use_zp else None, _op_kernel(x2d.shape[0], N, K, group_size)
 
 
 def w4a8_dense_apply(x2d: torch.Tensor, w_q: torch.Tensor, w_s: torch.Tensor,

@@ -400,6 +400,23 @@ def test_dense_ladder_and_env(monkeypatch):
         assert name in W._DENSE_KERNELS
 
 
+@pytest.mark.parametrize("env", [None, "4096", "2"])
+def test_dense_op_boundary(monkeypatch, env):
+    """A boundary set in the environment decides alone; unset, the tiles run where they lead."""
+    from w4a8_fp8_wmma import linear
+    monkeypatch.delenv("VLLM_ROCM_W4A8_DECODE_MAX_M", raising=False)
+    if env:
+        monkeypatch.setenv("VLLM_ROCM_W4A8_DECODE_MAX_M", env)
+    for M, N, K, lead in ((1, 28672, 4096, False), (16, 4096, 512, False), (17, 12288, 4096, True),
+                          (48, 12288, 4096, True), (64, 4096, 4096, False), (80, 4096, 4096, True),
+                          (300, 2048, 4096, True), (64, 16384, 128, False), (16, 28672, 512, True)):
+        gemv = not lead if env is None else M <= int(env)
+        x = torch.zeros(M, K, dtype=torch.float16, device="meta")
+        w = torch.zeros(N, K // 8, dtype=torch.int32, device="meta")
+        name = linear._dense_args(x, w, None, None, None, None, None, N, K, 128, False, 8, 0)[-1]
+        assert name == ("decode_gemv" if gemv else "prefill_wmma_ashuffle"), (M, N, K)
+
+
 def test_gptq_to_op_layout_from_the_format_definition():
     """AutoGPTQ qweight (K/8, N): word [k8, n] holds k = 8 k8 + j of column n in nibble j.
     Built element by element here, then converted and compared with the oracle's op-layout

@@ -8,6 +8,7 @@ import pytest
 import torch
 
 import w4a8_fp8_wmma as W
+from w4a8_fp8_wmma import _lib
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -118,6 +119,22 @@ def test_bf16_rows_equal_their_fp16_cast(M, N, K):
     a = torch.ops.vllm.w4a8_dense_apply(x, *args)
     b = torch.ops.vllm.w4a8_dense_apply(x.to(torch.float16), *args)
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 12288, 256), (300, 2048, 4096), (600, 4096, 1024)])
+def test_gemv_by_name(M, N, K, monkeypatch):
+    """The name "decode_gemv" runs the GEMV at any size: the same bits with a workspace, without
+    one (the rows then quantised in the kernel) and through the op with its boundary past M."""
+    x, w, s, z = _case(M, N, K, True, M + K)
+    want = W.mmq_fp8_gemm(x, w, s, kernel="decode_gemv", w_zeros=z)
+    bare = torch.empty_like(want)
+    _lib.check(_lib.lib.w4a8_mmq_fp8_gemm(
+        x.data_ptr(), M, K, w.data_ptr(), s.data_ptr(), z.data_ptr(), N, 128, W._DENSE_KERNELS["decode_gemv"],
+        0, bare.data_ptr(), None, 0, torch.cuda.current_stream().cuda_stream), "dense")
+    monkeypatch.setenv("VLLM_ROCM_W4A8_DECODE_MAX_M", "1000")
+    op = torch.ops.vllm.w4a8_dense_apply(x, w, s, z, None, None, None, N, K, 128, True, 0, 0)
+    tiles = W.mmq_fp8_gemm(x, w, s, kernel="prefill_wmma_ashuffle", w_zeros=z)
+    assert torch.equal(want, bare) and torch.equal(want, op) and not torch.equal(want, tiles)
 
 
 # no rows: an empty result and no launch, whichever kernel the sizes choose
