@@ -5,10 +5,10 @@
 //
 //   * the int32 words go into the MFMA as they are: a lane's 16 bytes are 32 E2M1 codes, the
 //     f8f6f4 MFMA's own fp4 operand, against e4m3 activations in natural k order;
-//   * scales that are powers of two (every MX checkpoint's: E8M0 converted to fp16 at load)
-//     become the MFMA's own block-scale operand, so a 128-wide K step is one MFMA per 16 x 16
+//   * scales that are powers of two (an MX checkpoint's: E8M0 converted to fp16 at load, exponents
+//     -14 to 15) become the MFMA's own block-scale operand, so a 128-wide K step is one MFMA per 16 x 16
 //     block that accumulates in place: no fold, no masked operands. A wave looks at the fp16
-//     fp16 scales as they come; a column with one that is not a normal positive power of two
+//     scales as they come; a column with one that is not a normal positive power of two
 //     is taken through the general form as well, which replaces its sums (one masked MFMA per
 //     group and the fp32 fold run += partial * scale, the arithmetic of the scalar kernel);
 //   * loads are coalesced along the weight rows (four lanes a row's 64 bytes of a step; 32
@@ -29,7 +29,10 @@
 // 103 / 132 -> 46 / 52 us, T = 256 346 / 246 -> 158 / 106, T = 1000 925 / 515 -> 422 / 190; the
 // layer with biases and swigluoai in one call (before: op by op) T = 8 380 -> 112 us, T = 1000
 // 967 -> 329. Scales that are no powers of two, gemm1 in 16- / 32- / 64-row blocks: T = 8
-// 102 / 114 / 133 -> 85 / 92 / 132 us, T = 1000 926 / 746 / 515 -> 645 / 428 / 536.
+// 102 / 114 / 133 -> 85 / 92 / 132 us, T = 1000 926 / 746 / 515 -> 645 / 428 / 536, but T = 1
+// 35 / 41 / 52 -> 32 / 50 / 104: fewer, larger work-groups than before, and their loads wait. With
+// such a scale in 2 of 100 columns both forms run: T = 1 35 / 41 / 52 -> 46 / 82 / 110, T = 1000
+// 925 / 738 / 506 -> 674 / 500 / 439.
 #include <algorithm>
 #include <type_traits>
 
@@ -274,8 +277,10 @@ __global__ void __launch_bounds__(256, 2) fp4_tiles_kernel(Params p, int nblocks
     // The general form: one masked MFMA per group and the fold run += partial * scale, for
     // fragments J0 .. J0 + NJ - 1 into run. Each wave reads the rows itself, without LDS: some
     // waves of the work-group may be past their work. Every row fragment takes part, live or
-    // not: with a uniform branch around each fragment's MFMAs the compiler moved a fold past
-    // the branch and left out the wait between an MFMA and the first read of its result.
+    // not: with a uniform branch around each fragment's MFMAs the compiler moved the folds past
+    // the branches, where it can leave out the wait between an MFMA and the next use of its
+    // result's registers (tests/test_cpu_mfma_waits.py walks the built code for that; the ring's
+    // branches guard MFMAs alone, whose results are read after its barriers).
     auto general_form = [&](auto j0c, auto njc, auto& run) __attribute__((always_inline)) {
         constexpr int J0 = decltype(j0c)::value, NJ = decltype(njc)::value;
 #pragma unroll

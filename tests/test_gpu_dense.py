@@ -53,8 +53,8 @@ def test_dense_apply_vs_oracle(M, asym):
 
 @pytest.mark.parametrize("M", [1, 40])
 def test_dense_long_k_vs_oracle(M):
-    """K = 6144 (48 groups): past the GEMV and streamed-K tables, so both names run the
-    general MFMA tiles."""
+    """K = 6144 (48 groups): the GEMV's waves do not split them evenly, so both names run the
+    split-K kernel."""
     r = np.random.default_rng(7050 + M)
     N, K, g = 384, 6144, 128
     nib, zp, sc = make_weights(r, N, K, g, True)
