@@ -22,8 +22,8 @@
 // The largest tile is bound by its LDS reads and VALU work (decode 3.25, fold 4 an MFMA) beside the
 // MFMAs, the small ones by the operations of one wave a SIMD: about 0.5 us a K group. Measured (us
 // a call of the op, zero-points, act-quant included; general or 64 x 256 tiles or GEMV -> these):
-// (N, K) = (4096, 12288) M = 2048 351 -> 154 (1.3 PF/s); (12288, 4096) M = 2048 267 -> 169, M = 48
-// 34 -> 26; (4096, 4096) M = 512 58 -> 34; (8192, 8192) M = 1 67 -> 39. On raw nibbles, with 32 x
+// (N, K) = (4096, 12288) M = 2048 351 -> 148 (1.4 PF/s); (12288, 4096) M = 2048 267 -> 158, M = 48
+// 34 -> 26; (4096, 4096) M = 512 58 -> 33; (8192, 8192) M = 1 67 -> 39. On raw nibbles, with 32 x
 // 128 to 128 x 256 tiles: 155, 153, 26, 31, 40.
 #include <algorithm>
 #include <type_traits>
@@ -89,13 +89,16 @@ __global__ void __launch_bounds__(C::kThreads, 2) wide_tiles_kernel(Params p, in
     const uint16_t* se = reinterpret_cast<const uint16_t*>(p.scales);
 
     // ---- staging: 32-bit byte offsets from the rows and the expert's slice ----
+    // place of row r in LDS: with the piece swizzle, equal pieces of sixteen rows lie in different
+    // banks (without it a third of the LDS cycles were conflicts: (12288, 4096) M = 2048 169 -> 158 us)
+    auto lrow = [](int r) __attribute__((always_inline)) { return r ^ ((r >> 3) & 1); };
     uint32_t aoff[C::ACH], boff[C::BCH], zoff[C::BCH];
     int adst[C::ACH], bdst[C::BCH][2], zsh[C::BCH];
 #pragma unroll
     for (int i = 0; i < C::ACH; ++i) {
         const int c = tid + i * C::kThreads, r = c >> 3, ch = c & 7;
         aoff[i] = (uint32_t)xrow(r) * (uint32_t)K + (uint32_t)ch * 16u;
-        adst[i] = r * kGroup + ((ch ^ (r & 7)) << 4);
+        adst[i] = lrow(r) * kGroup + ((ch ^ (r & 7)) << 4);
     }
 #pragma unroll
     for (int i = 0; i < C::BCH; ++i) {
@@ -105,7 +108,7 @@ __global__ void __launch_bounds__(C::kThreads, 2) wide_tiles_kernel(Params p, in
         zoff[i] = (uint32_t)(n >> 3) * (uint32_t)G * 4u;
         zsh[i] = 4 * (n & 7);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) bdst[i][h] = C::B + r * kGroup + (((2 * pc + h) ^ (r & 7)) << 4);
+        for (int h = 0; h < 2; ++h) bdst[i][h] = C::B + lrow(r) * kGroup + (((2 * pc + h) ^ (r & 7)) << 4);
     }
     u32x4 ar[2][C::ACH], br[2][C::BCH];
     uint32_t zr[2][ZP ? C::BCH : 1];
@@ -171,8 +174,8 @@ __global__ void __launch_bounds__(C::kThreads, 2) wide_tiles_kernel(Params p, in
 
     // One K group from its LDS slot (byte offset), gl its index in the chunk. The pieces of the
     // next group are decoded and stored between the MFMAs of the row fragments.
-    const int a_lane = (wm * MT * 16 + c16) * kGroup;
-    const int b_lane = C::B + (wn * NT * 16 + c16) * kGroup;
+    const int a_lane = (wm * MT * 16 + lrow(c16)) * kGroup;
+    const int b_lane = C::B + (wn * NT * 16 + lrow(c16)) * kGroup;
     const int p0 = ((2 * q) ^ (c16 & 7)) << 4, p1 = ((2 * q + 1) ^ (c16 & 7)) << 4;
     auto frag = [&](const uint8_t* r) __attribute__((always_inline)) {
         const u32x4 lo = *reinterpret_cast<const u32x4*>(r + p0), hi = *reinterpret_cast<const u32x4*>(r + p1);
