@@ -87,11 +87,12 @@ def _tiles_lead(M: int, N: int, K: int) -> bool:
 
 def _op_kernel(M: int, N: int, K: int, group_size: int) -> str:
     """The kernel name the op runs: a boundary set in the environment decides alone."""
-    name = dense_kernel_for(M, N, K, group_size)
-    if (name == "decode_gemv" and "VLLM_ROCM_W4A8_DECODE_MAX_M" not in os.environ
-            and _tiles_lead(M, N, K)):
-        return "prefill_wmma_ashuffle"
-    return name
+    if os.environ.get("VLLM_ROCM_W4A8_DECODE_MAX_M") is not None:
+        return dense_kernel_for(M, N, K, group_size)
+    # (up to the default boundary dense_kernel_for names the GEMV: one environment read a call)
+    few = group_size == 128 and M <= DECODE_MAX_M_DEFAULT and K % 128 == 0
+    name = "decode_gemv" if few else dense_kernel_for(M, N, K, group_size)
+    return "prefill_wmma_ashuffle" if name == "decode_gemv" and _tiles_lead(M, N, K) else name
 
 
 def _dense_args(x2d, w_q, w_s, w_zp, tri_bq, tri_s, tri_zp, N, K, group_size, zero_points,
