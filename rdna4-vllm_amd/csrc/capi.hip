@@ -107,8 +107,9 @@ int run_grouped(GroupedArgs& a, int64_t kernel, void* ws, size_t ws_bytes, hipSt
     if (wide) return split ? launch_dense_split(a, s) : launch_wide_tiles(a, s);
     // activation-resident tiles where the shape allows (the whole-layer prefill kernel, so
     // the op API and moe_apply share it), the streamed-K tiles otherwise. An ares work-group
-    // owns all N columns of its rows, so one expert (the dense GEMM) fills the chip only with
-    // >= 512 row tiles; below that the streamed-K tiles also split N.
+    // owns all N columns of its rows, so one expert fills the chip only with >= 512 row tiles;
+    // below that the streamed-K tiles also split N. (The dense op comes here with rows or weights
+    // of 2 GiB only.)
     const bool ares_fills = a.E > 1 || a.P >= 512 * 64;
     if (prefill && ares_fills &&
         prefill_ares_supported(a.K, a.N, a.group_size, a.e2m1, a.block_m, a.epi) &&
