@@ -68,9 +68,12 @@ int run_grouped(GroupedArgs& a, int64_t kernel, void* ws, size_t ws_bytes, hipSt
     float* gsum = w.take<float>((size_t)(a.x_rows * ((a.K + 127) / 128)));
     const bool have_ws = !(a.x_rows > 0 && ws == nullptr) && w.ok();
     const bool whole = gemv_whole_split(a.K, a.group_size);
-    // K groups that the GEMV's waves do not split evenly: the dense op runs its tiles under either
-    // name; without a workspace for the quantised rows the call is refused below
-    if (!whole && (dense || !have_ws)) gemv = false;
+    // K groups that the GEMV's waves do not split evenly: the tiles run under either name in the
+    // dense op and with many slots an expert, where they lead (E = 64, top-8, (K, N) = (2304, 1792),
+    // GEMV / tiles in us: 8 slots an expert 47 / 50 in 64-row blocks; 12 57 / 52, in 16-row blocks
+    // 47 / 49; 50 133 / 66 and 126 / 124; 125 266 / 150 and 264 / 250). Without a workspace for the
+    // quantised rows the call is refused below.
+    if (!whole && (dense || !have_ws || a.num_valid > (a.block_m == 16 ? 64 : 8) * a.E)) gemv = false;
     // identity-gathered inputs (gemm2 / scatter) have one row per padded row: skip padding.
     const bool filter = a.identity_gather && a.sorted_ids != nullptr;
     if (kernel == W4A8_MOE_KERNEL_GEMV && gemv) {

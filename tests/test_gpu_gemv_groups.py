@@ -51,6 +51,53 @@ def test_uneven_groups(G, asym, T, N, block_m):
     assert rows == T * k
 
 
+def _op(x, w, s, z, ids, block_m, kernel):
+    sti, eid, ntp = W.moe_align_block_size(ids, block_m, w.shape[0])
+    y = W.mmq_fp8_moe_gemm(x, w, s, sti, eid, ntp, ids.shape[1], block_m, kernel=kernel, w_zeros=z)
+    real = (sti < ids.numel()) & (torch.arange(sti.numel(), device=DEV) < ntp)
+    return y[real], sti[real].long() // ids.shape[1], eid.repeat_interleave(block_m)[real].long()
+
+
+@pytest.mark.parametrize("G", [5, 7, 10, 14, 18, 23])
+@pytest.mark.parametrize("block_m", [32, 64])
+def test_many_rows_in_a_block(G, block_m):
+    """Few slots an expert on average, 37 of them with one expert: several passes of 16 rows."""
+    E, T, N, K = 32, 37, 72, G * 128
+    g = torch.Generator(device=DEV).manual_seed(G + block_m)
+    words = lambda *s: torch.randint(-2**31, 2**31 - 1, s, generator=g, device=DEV,
+                                     dtype=torch.int64).to(torch.int32)
+    w, z = words(E, N, K // 8), words(E, N // 8, G)
+    s = (torch.rand((E, N, G), generator=g, device=DEV) * 0.015 + 0.005).to(torch.float16)
+    x = torch.randn((T, K), generator=g, device=DEV).to(torch.float16)
+    ids = torch.stack([torch.full((T,), 3), torch.randint(4, E, (T,))], 1).to(torch.int32).to(DEV)
+    got, tok, e = _op(x, w, s, z, ids, block_m, "gemv")
+    q, sc = W.act_quant_fp8(x)
+    xd = _e4m3(q) * sc.double()[:, None]
+    ref = torch.zeros_like(got, dtype=torch.float64)
+    for i in range(E):
+        at = (e == i).nonzero()[:, 0]
+        wd = _e4m3(W.dequant_fp8(w[i], 128, z[i])) * s[i].double().repeat_interleave(128, 1)
+        ref[at] = xd[tok[at]] @ wd.t()
+    assert got.shape[0] == 2 * T
+    assert float(((got.double() - ref).abs().amax(1) / ref.abs().amax(1)).max()) <= 2.0 ** -10
+
+
+@pytest.mark.parametrize("T,block_m", [(17, 32), (17, 64), (130, 16)])
+def test_many_slots_an_expert_run_the_tiles(T, block_m):
+    """Past 8 slots an expert (64 in 16-row blocks) both names run the tiles: the same bits."""
+    E, N, G = 4, 264, 7
+    g = torch.Generator(device=DEV).manual_seed(T + block_m)
+    words = lambda *s: torch.randint(-2**31, 2**31 - 1, s, generator=g, device=DEV,
+                                     dtype=torch.int64).to(torch.int32)
+    w, z = words(E, N, G * 16), words(E, N // 8, G)
+    s = (torch.rand((E, N, G), generator=g, device=DEV) * 0.015 + 0.005).to(torch.float16)
+    x = torch.randn((T, G * 128), generator=g, device=DEV).to(torch.float16)
+    ids = torch.rand((T, E), generator=g, device=DEV).argsort(1)[:, :2].to(torch.int32).contiguous()
+    assert torch.equal(_op(x, w, s, z, ids, block_m, "gemv")[0], _op(x, w, s, z, ids, block_m, "wmma")[0])
+    few = ids[:4].contiguous()   # 2 slots an expert: the GEMV
+    assert not torch.equal(_op(x[:4], w, s, z, few, block_m, "gemv")[0], _op(x[:4], w, s, z, few, block_m, "wmma")[0])
+
+
 # each split in gemm1 (gate and up, SiLU) and in gemm2 (slot outputs); one to four tiles a
 # work-group in gemm1, up to eight in gemm2
 @pytest.mark.parametrize("H,I", [(640, 128), (896, 640), (1152, 896), (1280, 1152), (1408, 1280), (1664, 1408),
@@ -109,5 +156,5 @@ def test_bounds_of_the_tiles_stay():
 
     assert tuple(call(64, 16).shape) == (16, 64)
     for N, block_m in ((64, 8), (2 ** 32 // K + 8, 16)):
-        with pytest.raises(RuntimeError, match="gemv grouped GEMM"):
+        with pytest.raises(RuntimeError, match="multiple of 16|2 GiB"):
             call(N, block_m)
